@@ -7,8 +7,6 @@ Kinds of case (`kind`):
             in one HIP graph as a serving engine captures its decode steps; the experts' slabs
             are in pinned host memory. Each pass copies the window's routing in and replays.
   eager     the same calls made from Python one by one, for an engine that runs without graphs.
-  prefetch  the decode window with the next layer's experts predicted (the prediction is right)
-            and staged along this layer (`prefetch(along=)`), beside a dense product per layer.
   policy    the policy step alone through the C entry points, one graph of a model's layers:
             `expert_cache_manage`, or `expert_cache_manage_remap` where slot ids are wanted.
   fused     `expert_cache_fused`: the policy step with both block alignments, for decode
@@ -82,8 +80,6 @@ def listed():
                 zipf=0.0, keep=0.5, **_BF16_BIG),
         # an engine without graphs: every layer's refresh is called from Python
         _decode("eager-1", 128, 96, 1, steps=1, windows=192, kind="eager", **_W8A8),
-        # next-layer prefetch beside a layer's dense work
-        _decode("prefetch-1", 128, 64, 1, kind="prefetch", **_W8A8),
         # the policy step of 48 layers: single-user decode
         _policy("policy-8", 128, 64, 1, 8),
         # 512 experts at 257 slots and 50 ids, LRU, the policy alone: odd slots, ragged ids
@@ -110,7 +106,7 @@ def draw(rng):
 
 
 def _drawn(rng):
-    kind = rng.choice(["decode", "decode", "prefetch", "eager", "policy", "policy", "fused",
+    kind = rng.choice(["decode", "decode", "decode", "eager", "policy", "policy", "fused",
                        "fused", "fused"])
     common = {"zipf": round(rng.uniform(0.7, 1.3), 2), "keep": round(rng.uniform(0.3, 0.8), 2)}
     if kind == "fused":
@@ -278,40 +274,17 @@ def _step_layers(caches, ids):
     return [c.refresh(i) for c, i in zip(caches, ids)]
 
 
-def _prefetch_window(caches, ids, x, weight):
-    """Decode steps with each layer's experts prefetched one layer ahead; the last layer
-    prefetches for the next step's first."""
-    outs, n, layers = [], ids.shape[0], len(caches)
-    for t in range(n):
-        for l in range(layers):
-            t1, l1 = (t, l + 1) if l + 1 < layers else (t + 1, 0)
-            if t1 < n and layers > 1:
-                caches[l1].prefetch(ids[t1, l1], along=caches[l])
-            torch.mm(x, weight)  # the layer's dense work
-            outs.append(caches[l].refresh(ids[t, l]))
-    return outs
-
-
 def prepare(case, seed):
     warm, windows = _ids(case, seed)
     s = SimpleNamespace(case=case, windows=windows, at=0, graph=None, out=None)
-    if case["kind"] in ("decode", "eager", "prefetch"):
+    if case["kind"] in ("decode", "eager"):
         s.caches = _caches(case, seed)
         for step in warm:
             _step_layers(s.caches, step)
         if case["kind"] != "eager":
             s.ids = windows[0].clone()
-            if case["kind"] == "prefetch":
-                gen = torch.Generator(device=DEV).manual_seed(seed + 1)
-                x, weight = (torch.randn(n, 4096, device=DEV, generator=gen).to(torch.bfloat16)
-                             for n in (256, 4096))
-                torch.mm(x, weight)
-                s.graph, s.out = _capture(lambda: torch.stack(
-                    _prefetch_window(s.caches, s.ids, x, weight)))
-                s.dense = (x, weight)
-            else:
-                s.graph, s.out = _capture(lambda: torch.stack(
-                    [o for step in s.ids for o in _step_layers(s.caches, step)]))
+            s.graph, s.out = _capture(lambda: torch.stack(
+                [o for step in s.ids for o in _step_layers(s.caches, step)]))
         s.state = {"%d.%s" % (l, f): getattr(c, f) for l, c in enumerate(s.caches)
                    for f in _Rows.FIELDS}
         s.state.update({"%d.%s" % (l, n): t for l, c in enumerate(s.caches)
@@ -434,14 +407,10 @@ def work(case):
         one += 2 * (4 * length + 4 * blocks + 4)
     elif case["kind"] != "policy" or case["remap"]:
         one += wide * mk
-    flops = 0.0
     if "w13" in case:
         one += 2 * inserts * (case["w13"] + case["w2"] + case["s13"] + case["s2"])
     n = case["layers"] * case["steps"]
-    if case["kind"] == "prefetch":
-        one += 2 * 4096 * (256 + 4096 + 256)
-        flops = 2.0 * n * 256 * 4096 * 4096
-    return {"bytes": float(one * n), "flops": flops}
+    return {"bytes": float(one * n), "flops": 0.0}
 
 
 def tolerance(case):
