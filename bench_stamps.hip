@@ -32,20 +32,21 @@ __device__ __forceinline__ void put_row(unsigned long long* row, unsigned long l
   *reinterpret_cast<u64x2*>(row) = u64x2{t0, t1};
 }
 
-// manage_k<CS, false, 4, true, TQ> with stamps
-template <int CS, int TQ>
-__global__ __launch_bounds__(kWave) void stamped_manage_k(ManageArgs a,
-                                                          unsigned long long* row) {
+// manage_k<W, GLOBAL_E, 4, true> with stamps
+template <int W, bool GLOBAL_E>
+__global__ __launch_bounds__(W* kWave) void stamped_manage_k(ManageArgs a,
+                                                             unsigned long long* row) {
   const unsigned long long t0 = clock_now();
-  __shared__ ManageLds<false> L;
+  __shared__ ManageLds<W, GLOBAL_E> L;
   args_in_sgprs(a);
-  long long idv[kIdRegs];
-  manage_step<CS, false, 4, TQ>(a, L, idv);
-  lds_sync();
-  remap_tail<false, 4>(a, L, idv);
+  long long idv;
+  manage_step<W, GLOBAL_E, 4>(a, L, idv);
+  step_sync<GLOBAL_E>();
+  remap_tail<W, GLOBAL_E, 4>(a, L, idv);
   __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
   const unsigned long long t1 = clock_now();
-  if (__lane_id() == 0) put_row(row, t0, t1);
+  if (threadIdx.x == 0) put_row(row, t0, t1);
 }
 
 // gather_k<kGatherUnroll, true, false, false> with stamps, one row per workgroup
@@ -66,18 +67,9 @@ __global__ __launch_bounds__(kWave) void stamped_empty_k(unsigned long long* row
   if (__lane_id() == 0) put_row(row, t0, clock_now());
 }
 
-template <int TQ>
-void launch_tq(const ManageArgs& a, unsigned long long* row, hipStream_t s) {
-  if (a.S <= 64)
-    hipLaunchKernelGGL((stamped_manage_k<1, TQ>), dim3(1), dim3(kWave), 0, s, a, row);
-  else if (a.S <= 128)
-    hipLaunchKernelGGL((stamped_manage_k<2, TQ>), dim3(1), dim3(kWave), 0, s, a, row);
-  else if (a.S <= 256)
-    hipLaunchKernelGGL((stamped_manage_k<4, TQ>), dim3(1), dim3(kWave), 0, s, a, row);
-  else if (a.S <= 512)
-    hipLaunchKernelGGL((stamped_manage_k<8, TQ>), dim3(1), dim3(kWave), 0, s, a, row);
-  else
-    hipLaunchKernelGGL((stamped_manage_k<16, TQ>), dim3(1), dim3(kWave), 0, s, a, row);
+template <int W, bool GLOBAL_E = false>
+void launch_waves(const ManageArgs& a, unsigned long long* row, hipStream_t s) {
+  hipLaunchKernelGGL((stamped_manage_k<W, GLOBAL_E>), dim3(1), dim3(W * kWave), 0, s, a, row);
 }
 
 }  // namespace
@@ -90,7 +82,7 @@ int stamped_manage_remap(const void* ids, int id_bytes, int mk, int E, int S, in
                          long long* slot_stamp, unsigned char* routed, long long* step,
                          int* miss, int* n_miss, int policy, int decay, void* out,
                          unsigned long long* row, hipStream_t stream) {
-  if (E <= 0 || E > kLdsExperts || S <= 0 || S > kMaxSlots || id_bytes != 4) return -1;
+  if (E <= 0 || E > 4096 || S <= 0 || S > kMaxSlots || id_bytes != 4) return -1;
   if (max_inserts < 0 || max_inserts > kMaxInserts || policy < 0 || policy > 1) return -1;
   if ((mk > 0 && out == nullptr) || row == nullptr) return -1;
   ManageArgs a;
@@ -111,12 +103,20 @@ int stamped_manage_remap(const void* ids, int id_bytes, int mk, int E, int S, in
   a.policy = policy;
   a.decay = decay;
   a.out = out;
-  switch (table_chunks(E)) {
-    case 1: launch_tq<1>(a, row, stream); break;
-    case 2: launch_tq<2>(a, row, stream); break;
-    case 4: launch_tq<4>(a, row, stream); break;
-    default: launch_tq<kTabRegs>(a, row, stream); break;
-  }
+  // the product's choice for decode steps: a thread for every expert and every slot
+  const int n = E > S ? E : S;
+  if (E > kLdsExperts)
+    launch_waves<16, true>(a, row, stream);
+  else if (n <= 64)
+    launch_waves<1>(a, row, stream);
+  else if (n <= 128)
+    launch_waves<2>(a, row, stream);
+  else if (n <= 256)
+    launch_waves<4>(a, row, stream);
+  else if (n <= 512)
+    launch_waves<8>(a, row, stream);
+  else
+    launch_waves<16>(a, row, stream);
   return (int)hipGetLastError();
 }
 

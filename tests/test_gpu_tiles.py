@@ -1,0 +1,109 @@
+"""Sizes at the edges of the policy step's and the alignments' work split, against the oracle.
+
+The policy step gives every expert and slot a thread of a workgroup of 1, 2, 4, 8 or 16
+waves, finds few victims one by one and many by sorting each wave's keys, and orders stamps by
+32-bit keys where they fit. The fused call runs in one workgroup up to 1024 ids and, above, in
+a workgroup per 1024 ids after the policy step. Whole values, so every comparison is exact.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_util as gu
+import oracle
+from test_gpu_fuzz import _device_state
+from test_gpu_remap_fused import _fused_call, _outs
+from test_oracle import align_lengths
+
+pytestmark = pytest.mark.gpu
+
+
+def _check_state(st, ref, tag):
+    for name in ("table", "map_cold", "slot_expert", "slot_stamp", "routed", "step", "miss",
+                 "n_miss"):
+        got, want = getattr(st, name)[0].cpu().numpy(), getattr(ref, name)
+        assert np.array_equal(got, want), f"{tag}: {name} at {gu.first_diff(got, want)}"
+
+
+def _step(st, ref, ids, mi, policy, decay, id64, tag):
+    dt = torch.int64 if id64 else torch.int32
+    d_ids = torch.as_tensor(ids, device=gu.DEV).to(dt)
+    out = torch.full_like(d_ids, -9)
+    rc = gu.manage_call(gu.lib(), st, 0, gu.ptr(d_ids), len(ids), st.E, mi, policy, decay,
+                        gu.ptr(out), 8 if id64 else 4)
+    assert rc == 0 and ref.manage(ids, st.E, mi, policy, decay) == 0
+    torch.cuda.synchronize()
+    _check_state(st, ref, tag)
+    assert np.array_equal(out.cpu().numpy(), oracle.remap(ids, ref.table)), tag
+
+
+@pytest.mark.parametrize("E,S", [(63, 64), (64, 65), (65, 3), (128, 129), (129, 128), (200, 256),
+                                 (257, 257), (512, 100), (513, 513), (900, 1024), (1024, 1000),
+                                 (1025, 1024), (2050, 40)])
+@pytest.mark.parametrize("policy", [0, 1])
+def test_policy_step_at_every_width(E, S, policy):
+    """Few inserts (1 .. 9 misses a step, across the line between the two victim searches) and
+    many, with few distinct stamps so that keys tie up to the slot, and ids past one and past
+    four of the workgroup's passes."""
+    rng = np.random.default_rng(E * 7 + S)
+    nhot = min(S, E)
+    hot, slots = rng.choice(E, nhot, replace=False), rng.choice(S, nhot, replace=False)
+    st, ref = _device_state(E, S, S, hot, slots, rng.integers(0, 5, size=S))
+    for t, misses in enumerate([0, 1, 2, 5, 6, 8, 9, 40, E, 1]):
+        table = ref.table
+        cold, warm = np.nonzero(table < 0)[0], np.nonzero(table >= 0)[0]
+        ids = np.concatenate([rng.permutation(cold)[:misses], rng.permutation(warm)[:3], [-1, E]])
+        ids = rng.permutation(ids).astype(np.int32)
+        if t == 4:
+            ids = np.resize(ids, 5 * 1024 + 3)
+        _step(st, ref, ids, S, policy, 3, t % 2 == 1, f"E={E} S={S} policy={policy} step {t}")
+
+
+@pytest.mark.parametrize("S,bits", [(40, 26), (100, 25), (200, 24), (500, 23), (1000, 22)])
+@pytest.mark.parametrize("policy", [0, 1])
+@pytest.mark.parametrize("misses", [3, 30])
+def test_stamps_at_the_edge_of_the_short_keys(S, bits, policy, misses):
+    """Stamps on both sides of the largest that has a 32-bit key (`bits` bits above the slot),
+    counted from zero under LFU and back from the step under LRU, beside empty slots."""
+    E = min(1024, S + 60)
+    rng = np.random.default_rng(S + policy)
+    hot, slots = rng.choice(E, S - 4, replace=False), rng.choice(S, S - 4, replace=False)
+    top = 1 << bits
+    for far in (False, True):
+        edge = np.arange(top - 12, top + 4 if far else top - 6)
+        stamps = rng.choice(np.concatenate([[0, 1, 2], edge]), size=S)
+        if policy == 0:
+            stamps = np.where(stamps > 2, (1 << 40) - stamps, stamps * (1 << 39) if far else 0)
+        st, ref = _device_state(E, S, S, hot, slots, stamps)
+        st.step[0] = 1 << 40
+        ref.step[:] = 1 << 40
+        for t in range(3):
+            cold = np.nonzero(ref.table < 0)[0]
+            ids = rng.permutation(cold)[:misses].astype(np.int32)
+            _step(st, ref, ids, S, policy, 0, False, f"S={S} policy={policy} far={far} step {t}")
+
+
+@pytest.mark.parametrize("mk", [1, 64, 65, 255, 256, 257, 1023, 1024, 1025, 2048, 2051, 5000])
+@pytest.mark.parametrize("E,S,bs", [(7, 3, 1), (128, 64, 16), (200, 257, 12), (1024, 1024, 64)])
+def test_fused_at_the_workgroups_edges(mk, E, S, bs):
+    """From one id to several workgroups' ids, with padding and out-of-range ids and a few
+    popular experts; the ids start on a 16-byte boundary and 4 bytes past one."""
+    rng = np.random.default_rng(mk + E)
+    L, NB = align_lengths(mk, E, bs)
+    st, ref = gu.Layers(1, E, S), oracle.State(E, S)
+    for t in range(3):
+        ids = rng.integers(-2, E + 2, size=mk).astype(np.int32)
+        ids[rng.random(mk) < 0.3] = rng.integers(0, min(E, 4))
+        outs = _outs(L, NB)
+        d_ids = torch.zeros(mk + 1, dtype=torch.int32, device=gu.DEV)
+        d_ids = d_ids[1:] if t == 1 else d_ids[:mk]
+        d_ids.copy_(torch.as_tensor(ids))
+        assert _fused_call(gu.lib(), st, d_ids, mk, bs, L, NB, outs) == 0
+        rc, want = ref.fused(ids, min(E, mk), S, bs, L, NB)
+        assert rc == 0
+        torch.cuda.synchronize()
+        for k, v in want.items():
+            assert np.array_equal(outs[k].cpu().numpy(), v), (t, k)
+        _check_state(st, ref, f"mk={mk} step {t}")

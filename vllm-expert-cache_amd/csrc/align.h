@@ -1,5 +1,5 @@
 // expert_cache_fused on gfx950: the LRU policy step followed by both moe_align_block_size
-// outputs, in one wavefront (kernels/expert_cache.hip:431-588 semantics).
+// outputs (kernels/expert_cache.hip:431-588 semantics).
 //
 // The policy half is manage_step with policy 0 and no decay (a hit and an install both stamp
 // the current step). The align half buckets every routing id against the updated table --
@@ -7,16 +7,30 @@
 // multiple of the block size, scans, and places each id at its bucket offset plus its rank
 // among the earlier ids of the same bucket, so the output is in token order within every
 // bucket for every mk (the reference is token-ordered for mk <= 256 and unordered above).
-// Below each side's padded total the outputs are built in LDS (padding, block expert ids,
-// then the placed ids) and copied out with coalesced stores; past it the defaults go
-// straight to memory. No output position is written twice, so no fence is needed; outputs
-// too large for LDS are filled with their defaults in memory first and fenced.
+//
+// An id's rank is found without a pass over earlier ids: its lane's rank among the lanes of
+// its wave with the same bucket (wave_match), plus the counts of the earlier waves, which
+// each wave leaves in its own row of a small count matrix in LDS, plus, where several
+// workgroups share the ids, the count of the workgroup's earlier ids. No output position is
+// written twice (an id, its bucket's padding, or the default past the padded total), so
+// nothing is staged and no store is waited for.
+//
+//  * fused_k, up to kFusedIds ids: the policy step and both alignments in one workgroup,
+//    one id, one expert and one slot a thread.
+//  * align_k, more ids: a workgroup per 1024 ids, after a launch of the policy step alone.
+//    Each workgroup counts the ids before and after its own itself (they come from the L2),
+//    which costs less than the node or the cross-XCD handoff that sharing the counts would.
+//
+// Measured on MI355X, us a launch in a graph, against the same work in one wave that staged
+// its output in LDS: 8 ids (128 experts, 64 slots, block 16) 4.7 -> 3.9; 512 ids (256, 128,
+// 16) 12.6 -> 7.3; 16384 ids (128, 64, 64) 232 -> 15.6.
 #pragma once
 #include "manage.h"
 
 namespace ec {
 
 constexpr int kMaxAlignExperts = 1024;
+constexpr int kFusedIds = 1024;  // most ids of the one-workgroup kernel: one a thread
 
 struct AlignArgs {
   int bs, L, NB;
@@ -28,22 +42,26 @@ struct AlignArgs {
   int* npad_cold;
 };
 
-// Per side, the ids and block expert ids below the padded total are built in LDS and
-// copied out once when they fit in kStage ints (decode and chunked-prefill shapes).
-constexpr int kStage = 10240;
-
+// Buckets are slots 0 .. S-1 (hot), then S + e for expert e (cold): at most 2T.
+template <int W>
 struct AlignLds {
-  int cur_h[kMaxSlots + 1];          // counts, then placement cursors, per slot bucket
-  int cur_c[kMaxAlignExperts + 1];   // same per expert bucket
-  unsigned long long lanes[kMaxSlots + kMaxAlignExperts];  // per bucket key: lanes of a block
-  alignas(16) int stage[2][kStage];  // per side: sorted, then expert ids from round4(n)
+  static constexpr int T = W * kWave;
+  unsigned short cnt[W][2 * T];  // ids per bucket of each wave, then of the waves before it
+  int start[2 * T];  // position of the workgroup's first id of the bucket
+  int end[2 * T];    // position past the bucket's last id
+  int wsum[2][W];
 };
 
-// Combined bucket key of one routing id: slot s (hot), kMaxSlots + e (cold), -1 (skipped).
+// What one workgroup's thread needs after align_place: the padded totals of both sides.
+struct AlignTotals {
+  int hot, cold;
+};
+
+// Bucket of one routing id, -1 for padding and out-of-range ids.
 __device__ __forceinline__ int align_key(int e, int E, int S, const int* tab) {
   if (e < 0 || e >= E) return -1;
   const int s = tab[e];
-  return ((unsigned)s < (unsigned)S) ? s : kMaxSlots + e;
+  return ((unsigned)s < (unsigned)S) ? s : S + e;
 }
 
 // x / bs for the wave-uniform block size: a shift for powers of two (vLLM's block sizes).
@@ -55,220 +73,241 @@ struct BlockDiv {
   __device__ __forceinline__ int pad(int x) const { return div(x + bs - 1) * bs; }
 };
 
-// Exclusive scan of block-padded counts, 64 buckets per chunk (bucket c*64 + lane in chunk
-// c), kept in registers: ex[c] is the bucket's first position, pc[c] its padded count.
-// Returns the padded total. NC chunks cover nb buckets; chunks past nb are skipped on a
-// uniform branch. The count reads of every chunk are issued before the first scan.
-template <int NC>
-__device__ __forceinline__ int padded_scan(const int* cnt, int nb, BlockDiv d, int (&ex)[NC],
-                                           int (&pc)[NC]) {
-  const int lane = __lane_id();
-  int raw[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) raw[c] = cnt[min(c * kWave + lane, nb - 1)];
-  int run = 0;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    pc[c] = c * kWave + lane < nb ? d.pad(raw[c]) : 0;
-    ex[c] = run;
-    if (c * kWave < nb) {
-      const int incl = wave_incl_scan(pc[c]);
-      ex[c] = run + incl - pc[c];
-      run += __builtin_amdgcn_readlane(incl, kWave - 1);
-    }
-  }
-  return run;
-}
-
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-// dst[from, to) = v over the wave; 16-byte stores when dst is 16-byte aligned.
-__device__ __forceinline__ void fill_i32(int* dst, int from, int to, int v) {
-  const int lane = __lane_id();
+// dst[from, to) = v over `n` threads of which this is number `me`; 16-byte stores when dst is
+// 16-byte aligned.
+__device__ __forceinline__ void fill_i32(int* dst, int from, int to, int v, int me, int n) {
   if (from >= to) return;
   if ((reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
     const int a0 = min((from + 3) & ~3, to);
     const int a1 = a0 + ((to - a0) & ~3);
-    if (from + lane < a0) dst[from + lane] = v;
-    for (int p = a0 + 4 * lane; p < a1; p += 4 * kWave)
+    if (me < a0 - from) dst[from + me] = v;
+    for (long long p = a0 + 4ll * me; p < a1; p += 4ll * n)
       *reinterpret_cast<i32x4*>(dst + p) = i32x4{v, v, v, v};
-    if (a1 + lane < to) dst[a1 + lane] = v;
+    if (me < to - a1) dst[a1 + me] = v;
   } else {
-    for (int p = from + lane; p < to; p += kWave) dst[p] = v;
+    for (long long p = from + me; p < to; p += n) dst[p] = v;
   }
 }
 
-// dst[0, n) = src[0, n) from 16-byte aligned LDS; 16-byte stores when dst is aligned.
-__device__ __forceinline__ void copy_out(int* dst, const int* src, int n) {
-  const int lane = __lane_id();
-  if ((reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-    const int n4 = n & ~3;
-    for (int p = 4 * lane; p < n4; p += 4 * kWave)
-      *reinterpret_cast<i32x4*>(dst + p) = *reinterpret_cast<const i32x4*>(src + p);
-    if (n4 + lane < n) dst[n4 + lane] = src[n4 + lane];
-  } else {
-    for (int p = lane; p < n; p += kWave) dst[p] = src[p];
-  }
+// Clears the rows of the count matrix that `waves` waves fill; the caller syncs.
+template <int W>
+__device__ __forceinline__ void align_clear(AlignLds<W>& A, int waves, int buckets) {
+  constexpr int T = W * kWave;
+  unsigned* rows = reinterpret_cast<unsigned*>(A.cnt);
+  if (2 * (int)threadIdx.x < buckets)
+    for (int w = 0; w < waves; ++w) rows[w * T + threadIdx.x] = 0;
 }
 
-// Expert id of every block of every non-empty bucket, from the scan held in registers.
-template <int NC>
-__device__ __forceinline__ void fill_eids(const int (&ex)[NC], const int (&pc)[NC], int nb,
-                                          BlockDiv d, int NB, int* eids) {
-  const int lane = __lane_id();
+// Places id `i` of bucket `kk` (-1: none) for every thread of the workgroup, whose ids are
+// consecutive and lie in its first `waves` waves. The count matrix is clear. With PART the
+// workgroup holds only some of the ids: on entry A.start and A.end hold, per bucket, the
+// counts of the ids before and after its own. On return A.end and, per bucket, A.start are
+// positions as declared (behind the sync made here).
+template <int W, bool PART>
+__device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<W>& A, int E,
+                                                   int S, BlockDiv d, int kk, int i,
+                                                   int waves) {
+  const int tid = threadIdx.x, lane = __lane_id(), wave = wave_index();
+  int rank = 0;
+  if (wave < waves) {
+    const unsigned long long m = wave_match(kk, 32 - __clz(S + E - 1));
+    rank = __popcll(m & lanes_below());
+    // the bucket's last lane in the wave leaves the wave's count
+    if (kk >= 0 && (m >> lane) == 1ull) A.cnt[wave][kk] = (unsigned short)(rank + 1);
+  }
+  lds_sync();
+  // thread b: slot bucket b and expert bucket S + b
+  int n[2] = {0, 0}, before[2] = {0, 0};
+  const int size[2] = {S, E};
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int b = c * kWave + lane;
-    if (b < nb) {
-      const int q1 = min(d.div(ex[c] + pc[c]), NB);
-      for (int q = d.div(ex[c]); q < q1; ++q) eids[q] = b;
+  for (int h = 0; h < 2; ++h) {
+    const int b = tid + (h ? S : 0);
+    if (tid < size[h]) {
+      if (waves == 1) {
+        n[h] = A.cnt[0][b];
+        A.cnt[0][b] = 0;
+      } else {
+        for (int w0 = 0; w0 < waves; w0 += 4) {
+          int c[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) c[q] = w0 + q < waves ? A.cnt[min(w0 + q, W - 1)][b] : 0;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (w0 + q < waves) A.cnt[min(w0 + q, W - 1)][b] = (unsigned short)n[h];
+            n[h] += c[q];
+          }
+        }
+      }
+      if constexpr (PART) {
+        before[h] = A.start[b];
+        n[h] += before[h] + A.end[b];
+      }
     }
   }
-}
-
-// Places the ids of one block of 64 (lane -> id i, bucket key kk or -1) at their bucket's
-// cursor plus their rank among the earlier ids of the same bucket in the block, so every
-// bucket is in token order. The lanes sharing a bucket are found by an atomic OR of lane
-// bits into the bucket's mask (order-free, so deterministic; every mask starts the block at
-// zero); a lane's rank is the popcount of the mask below it. The bucket's last lane moves
-// the cursor and clears the mask for the next block.
-__device__ __forceinline__ void place_block(const AlignArgs& g, AlignLds& A, int kk, int i,
-                                            int* sorted_hot, int* sorted_cold) {
-  const int lane = __lane_id();
-  if (kk >= 0) atomicOr(&A.lanes[kk], 1ull << lane);
-  lds_sync();
-  const int kc = kk < 0 ? 0 : kk;
-  int* cur = kc >= kMaxSlots ? &A.cur_c[kc - kMaxSlots] : &A.cur_h[kc];
-  const unsigned long long m = A.lanes[kc];
-  const int c0 = *cur;
-  if (kk >= 0) {
-    const int pos = c0 + __popcll(m & lanes_below());
-    int* sorted = kk >= kMaxSlots ? sorted_cold : sorted_hot;
-    if (pos < g.L) sorted[pos] = i;
-    if ((m >> lane) == 1ull) {
-      *cur = c0 + __popcll(m);
-      A.lanes[kc] = 0ull;
+  // exclusive scans of the padded counts of both sides over the threads
+  const int padded[2] = {d.pad(n[0]), d.pad(n[1])};
+  int first[2], total[2];
+  int scan[2] = {wave_incl_scan(padded[0]), wave_incl_scan(padded[1])};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    first[h] = scan[h] - padded[h];
+    total[h] = __builtin_amdgcn_readlane(scan[h], kWave - 1);
+    if constexpr (W > 1) {
+      if (lane == 0) A.wsum[h][wave] = total[h];
     }
   }
-  lds_sync();
-}
-
-// Every id in token order: the first kIdRegs blocks from the keys held in registers, the
-// rest from memory.
-__device__ __forceinline__ void place_ids(const ManageArgs& a, const AlignArgs& g,
-                                          const ManageLds<false>& L, AlignLds& A,
-                                          const int (&key)[kIdRegs], int* sorted_hot,
-                                          int* sorted_cold) {
-  const int lane = __lane_id();
-  const int mk = a.mk;
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k)
-    if (k * kWave < mk) place_block(g, A, key[k], lane + k * kWave, sorted_hot, sorted_cold);
-  const int* ids = reinterpret_cast<const int*>(a.ids);
-  for (int base = kIdRegs * kWave; base < mk; base += kWave) {
-    const int i = base + lane;
-    const int kk = i < mk ? align_key(ids[i], a.E, a.S, L.tab) : -1;
-    place_block(g, A, kk, i, sorted_hot, sorted_cold);
-  }
-}
-
-template <int CS, int TQ>
-__device__ __forceinline__ void align_tail(const ManageArgs& a, const AlignArgs& g,
-                                           const ManageLds<false>& L, AlignLds& A,
-                                           const long long (&idv)[kIdRegs]) {
-  // chunks of 64 buckets per side: the slots per lane cover S; the table chunks cover E up
-  // to 512, and 16 chunks cover the rest (E <= kMaxAlignExperts)
-  constexpr int CC = TQ == kTabRegs ? kMaxAlignExperts / kWave : TQ;
-  const int lane = __lane_id();
-  const int E = a.E, S = a.S, mk = a.mk;
-  const BlockDiv d(g.bs);
-  const int* ids = reinterpret_cast<const int*>(a.ids);
-
-  // bucket key of every id held in registers (the table lookups issued together)
-  int key[kIdRegs];
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k)
-    key[k] = lane + k * kWave < mk ? align_key((int)idv[k], E, S, L.tab) : -1;
-  for (int b = lane; b < S; b += kWave) A.cur_h[b] = 0;
-  for (int b = lane; b < E; b += kWave) A.cur_c[b] = 0;
-  lds_sync();
-  // counts per bucket; each used bucket's lane mask starts at zero for the placement
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k) {
-    const int kk = key[k];
-    if (kk >= kMaxSlots)
-      atomicAdd(&A.cur_c[kk - kMaxSlots], 1);
-    else if (kk >= 0)
-      atomicAdd(&A.cur_h[kk], 1);
-    if (kk >= 0) A.lanes[kk] = 0ull;
-  }
-  for (int i = lane + kIdRegs * kWave; i < mk; i += kWave) {
-    const int kk = align_key(ids[i], E, S, L.tab);
-    if (kk >= kMaxSlots)
-      atomicAdd(&A.cur_c[kk - kMaxSlots], 1);
-    else if (kk >= 0)
-      atomicAdd(&A.cur_h[kk], 1);
-    if (kk >= 0) A.lanes[kk] = 0ull;
-  }
-  lds_sync();
-  int exh[CS], pch[CS], exc[CC], pcc[CC];
-  const int tot_h = padded_scan(A.cur_h, S, d, exh, pch);
-  const int tot_c = padded_scan(A.cur_c, E, d, exc, pcc);
-  if (lane == 0) {
-    g.npad_hot[0] = tot_h;
-    g.npad_cold[0] = tot_c;
-  }
-  // placement cursors start at each bucket's first position (the counts were read above)
-#pragma unroll
-  for (int c = 0; c < CS; ++c)
-    if (c * kWave + lane < S) A.cur_h[c * kWave + lane] = exh[c];
-#pragma unroll
-  for (int c = 0; c < CC; ++c)
-    if (c * kWave + lane < E) A.cur_c[c * kWave + lane] = exc[c];
-
-  // Every position below a side's padded total is an id or its bucket's padding, every
-  // block below it belongs to a bucket; past it the outputs hold mk and -1.
-  const int nh = min(tot_h, g.L), nc = min(tot_c, g.L);
-  const int qh = min(d.div(tot_h), g.NB), qc = min(d.div(tot_c), g.NB);
-  const int oh = (nh + 3) & ~3, oc = (nc + 3) & ~3;
-  if (oh + qh <= kStage && oc + qc <= kStage) {
-    int* sh = A.stage[0];
-    int* sc = A.stage[1];
-    fill_i32(sh, 0, nh, mk);
-    fill_i32(sc, 0, nc, mk);
-    fill_eids(exh, pch, S, d, g.NB, sh + oh);
-    fill_eids(exc, pcc, E, d, g.NB, sc + oc);
-    fill_i32(g.sorted_hot, nh, g.L, mk);
-    fill_i32(g.sorted_cold, nc, g.L, mk);
-    fill_i32(g.eids_hot, qh, g.NB, -1);
-    fill_i32(g.eids_cold, qc, g.NB, -1);
+  if constexpr (W > 1) {
     lds_sync();
-    place_ids(a, g, L, A, key, sh, sc);  // ends with an LDS sync
-    copy_out(g.sorted_hot, sh, nh);
-    copy_out(g.eids_hot, sh + oh, qh);
-    copy_out(g.sorted_cold, sc, nc);
-    copy_out(g.eids_cold, sc + oc, qc);
-  } else {
-    fill_i32(g.sorted_hot, 0, g.L, mk);
-    fill_i32(g.eids_hot, 0, g.NB, -1);
-    fill_i32(g.sorted_cold, 0, g.L, mk);
-    fill_i32(g.eids_cold, 0, g.NB, -1);
-    mem_sync();  // the defaults are written before any entry below lands on them
-    fill_eids(exh, pch, S, d, g.NB, g.eids_hot);
-    fill_eids(exc, pcc, E, d, g.NB, g.eids_cold);
-    place_ids(a, g, L, A, key, g.sorted_hot, g.sorted_cold);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int b;
+      wave_sums<W>(A.wsum[h], wave, b, total[h]);
+      first[h] += b;
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (tid < size[h]) {
+      const int b = tid + (h ? S : 0);
+      A.start[b] = first[h] + before[h];
+      A.end[b] = first[h] + n[h];
+    }
+  }
+  lds_sync();
+  if (kk >= 0) {
+    const int pos = A.start[kk] + A.cnt[wave][kk] + rank;
+    int* sorted = kk < S ? g.sorted_hot : g.sorted_cold;
+    if (pos < g.L) sorted[pos] = i;
+  }
+  return {total[0], total[1]};
+}
+
+// The padding of each bucket (mk) and its blocks' expert ids, a wave per bucket of the
+// launch's `nwaves`, this one being number `me`. `from` is the bucket's first position.
+template <int W>
+__device__ __forceinline__ void align_pad(const AlignArgs& g, const AlignLds<W>& A, int E,
+                                          int S, int mk, BlockDiv d, int me, int nwaves,
+                                          const int* from) {
+  const int lane = __lane_id();
+  for (int b = me; b < S + E; b += nwaves) {
+    const int p0 = from[b], p1 = A.end[b];
+    if (p0 == p1) continue;
+    const int p2 = p0 + d.pad(p1 - p0);
+    int* sorted = b < S ? g.sorted_hot : g.sorted_cold;
+    int* eids = b < S ? g.eids_hot : g.eids_cold;
+    const int id = b < S ? b : b - S;
+    for (int p = p1 + lane; p < min(p2, g.L); p += kWave) sorted[p] = mk;
+    const int q1 = min(d.div(p2), g.NB);
+    for (int q = d.div(p0) + lane; q < q1; q += kWave) eids[q] = id;
   }
 }
 
-template <int CS, int TQ>
-__global__ __launch_bounds__(kWave) void fused_k(ManageArgs a, AlignArgs g) {
-  __shared__ ManageLds<false> L;
-  __shared__ AlignLds A;
+// Past the padded totals the outputs hold mk and -1.
+__device__ __forceinline__ void align_rest(const AlignArgs& g, int mk, BlockDiv d,
+                                           AlignTotals t, int me, int n) {
+  if (me == 0) {
+    g.npad_hot[0] = t.hot;
+    g.npad_cold[0] = t.cold;
+  }
+  fill_i32(g.sorted_hot, min(t.hot, g.L), g.L, mk, me, n);
+  fill_i32(g.sorted_cold, min(t.cold, g.L), g.L, mk, me, n);
+  fill_i32(g.eids_hot, min(d.div(t.hot), g.NB), g.NB, -1, me, n);
+  fill_i32(g.eids_cold, min(d.div(t.cold), g.NB), g.NB, -1, me, n);
+}
+
+// One workgroup: T >= E, S and mk.
+template <int W>
+__global__ __launch_bounds__(W* kWave) void fused_k(ManageArgs a, AlignArgs g) {
+  constexpr int T = W * kWave;
+  __shared__ ManageLds<W, false> L;
+  __shared__ AlignLds<W> A;
+  // per side, the bucket of each block below the padded total: no more blocks than ids
+  __shared__ unsigned short block[2][T];
   args_in_sgprs(a);
-  long long idv[kIdRegs];
-  manage_step<CS, false, 4, TQ>(a, L, idv);
+  const int tid = threadIdx.x;
+  const int E = a.E, S = a.S, mk = a.mk, waves = (mk + kWave - 1) / kWave;
+  const BlockDiv d(g.bs);
+  align_clear<W>(A, max(waves, 1), S + E);
+  long long idv;
+  manage_step<W, false, 4>(a, L, idv);
   lds_sync();
-  align_tail<CS, TQ>(a, g, L, A, idv);
+  const int kk = align_key((int)idv, E, S, L.tab);
+  const AlignTotals t = align_place<W, false>(g, A, E, S, d, kk, tid, max(waves, 1));
+  align_rest(g, mk, d, t, tid, T);
+  // thread b names the blocks of its two buckets
+  if (tid < S)
+    for (int q = d.div(A.start[tid]), q1 = d.div(A.end[tid] + g.bs - 1); q < q1; ++q)
+      block[0][q] = (unsigned short)tid;
+  if (tid < E)
+    for (int q = d.div(A.start[S + tid]), q1 = d.div(A.end[S + tid] + g.bs - 1); q < q1; ++q)
+      block[1][q] = (unsigned short)tid;
+  lds_sync();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int total = h ? t.cold : t.hot;
+    const int* end = A.end + (h ? S : 0);
+    int* sorted = h ? g.sorted_cold : g.sorted_hot;
+    int* eids = h ? g.eids_cold : g.eids_hot;
+    const int q1 = min(d.div(total), g.NB);
+    for (int q = tid; q < q1; q += T) eids[q] = block[h][q];
+    const int p1 = min(total, g.L);
+    for (int p = tid; p < p1; p += T)
+      if (p >= end[block[h][d.div(p)]]) sorted[p] = mk;
+  }
+}
+
+// A workgroup per 1024 ids, against the table as it is.
+__global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, int S,
+                                                const int* table, AlignArgs g) {
+  constexpr int W = 16, T = W * kWave;
+  __shared__ AlignLds<W> A;
+  __shared__ int from[2 * T];           // first position of each bucket
+  __shared__ unsigned short bucket[T];  // of each expert
+  const int tid = threadIdx.x, part = blockIdx.x, parts = gridDim.x;
+  const int first = part * T;
+  const BlockDiv d(g.bs);
+  if (tid < E) {
+    const int s = table[tid];
+    bucket[tid] = (unsigned short)((unsigned)s < (unsigned)S ? s : S + tid);
+  }
+  align_clear<W>(A, W, S + E);
+  A.start[tid] = A.start[T + tid] = A.end[tid] = A.end[T + tid] = 0;
+  lds_sync();
+  // ids of the other workgroups, counted per bucket: before this one's, and after
+  auto count = [&](int e, int i) {
+    if (e >= 0 && e < E) atomicAdd(&(i < first ? A.start : A.end)[bucket[e]], 1);
+  };
+  const int mine = first + tid < mk ? ids[first + tid] : -1;
+  if ((reinterpret_cast<uintptr_t>(ids) & 15) == 0) {
+    // four ids a load; `first` is a multiple of four and only the last workgroup's ids end
+    // at mk, so no vector straddles a boundary except the one cut off here
+    const int n4 = mk & ~3;
+    for (int i = 4 * tid; i < n4; i += 4 * T) {
+      if (i >= first && i < first + T) continue;
+      const i32x4 e = *reinterpret_cast<const i32x4*>(ids + i);
+      count(e.x, i);
+      count(e.y, i);
+      count(e.z, i);
+      count(e.w, i);
+    }
+    const int i = n4 + tid;
+    if (i < mk && (i < first || i >= first + T)) count(ids[i], i);
+  } else {
+    for (int i = tid; i < mk; i += T)
+      if (i < first || i >= first + T) count(ids[i], i);
+  }
+  lds_sync();
+  // positions of the buckets' starts: align_place leaves this workgroup's own in A.start
+  int before[2] = {tid < S ? A.start[tid] : 0, tid < E ? A.start[S + tid] : 0};
+  const int kk = mine >= 0 && mine < E ? bucket[mine] : -1;
+  const AlignTotals t = align_place<W, true>(g, A, E, S, d, kk, first + tid, W);
+  if (tid < S) from[tid] = A.start[tid] - before[0];
+  if (tid < E) from[S + tid] = A.start[S + tid] - before[1];
+  lds_sync();
+  align_rest(g, mk, d, t, first + tid, parts * T);
+  align_pad<W>(g, A, E, S, mk, d, part * W + wave_index(), parts * W, from);
 }
 
 }  // namespace ec

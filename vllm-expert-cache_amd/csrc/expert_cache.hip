@@ -2,9 +2,12 @@
 //
 // Argument checks run on the host before any HIP call and return -1, exactly where the
 // reference's C-ABI does (kernels/expert_cache.hip:596-598, :616-618, :631-634); otherwise
-// each entry point launches one kernel on the caller's stream and returns hipGetLastError().
+// each entry point launches one kernel (the fused one, for prefill chunks, two) on the
+// caller's stream and returns hipGetLastError().
 // The library keeps no state and allocates nothing.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "../../include/expert_cache.h"
 #include "align.h"
@@ -28,123 +31,80 @@ bool manage_args_bad(int E, int S, int max_inserts, int policy) {
   return false;
 }
 
-// Slots per lane (CS) by S, and table chunks held in registers (TQ) by E.
-template <int IDB, bool REMAP, int TQ>
-int launch_manage_tq(const ManageArgs& a, hipStream_t stream) {
-  const dim3 grid(1), block(kWave);
-  if (a.S <= 64) {
-    hipLaunchKernelGGL((manage_k<1, false, IDB, REMAP, TQ>), grid, block, 0, stream, a);
-  } else if (a.S <= 128) {
-    hipLaunchKernelGGL((manage_k<2, false, IDB, REMAP, TQ>), grid, block, 0, stream, a);
-  } else if (a.S <= 256) {
-    hipLaunchKernelGGL((manage_k<4, false, IDB, REMAP, TQ>), grid, block, 0, stream, a);
-  } else if (a.S <= 512) {
-    hipLaunchKernelGGL((manage_k<8, false, IDB, REMAP, TQ>), grid, block, 0, stream, a);
-  } else {
-    hipLaunchKernelGGL((manage_k<16, false, IDB, REMAP, TQ>), grid, block, 0, stream, a);
+// Waves of the policy step's workgroup: one thread for every expert and every slot, and a
+// quarter of one for every id (prefill chunks route far more ids than there are experts).
+int waves_for(int E, int S, int ids) {
+  const int n = E > S ? E : S;
+  const int threads = ids / 4 > n ? ids / 4 : n;
+  int w = 1;
+  while (w < 16 && w * kWave < threads) w *= 2;
+  return w;
+}
+
+// Calls f with the number of waves as a compile-time constant.
+template <class F>
+void with_waves(int w, F&& f) {
+  switch (w) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 4: f(std::integral_constant<int, 4>()); break;
+    case 8: f(std::integral_constant<int, 8>()); break;
+    default: f(std::integral_constant<int, 16>()); break;
   }
-  return (int)hipGetLastError();
 }
 
 template <int IDB, bool REMAP>
 int launch_manage(const ManageArgs& a, hipStream_t stream) {
   if (a.E > kLdsExperts) {
-    hipLaunchKernelGGL((manage_k<16, true, IDB, REMAP, kTabRegs>), dim3(1), dim3(kWave), 0,
-                       stream, a);
-    return (int)hipGetLastError();
+    hipLaunchKernelGGL((manage_k<16, true, IDB, REMAP>), dim3(1), dim3(16 * kWave), 0, stream,
+                       a);
+  } else {
+    with_waves(waves_for(a.E, a.S, a.mk), [&](auto w) {
+      hipLaunchKernelGGL((manage_k<w(), false, IDB, REMAP>), dim3(1), dim3(w() * kWave), 0,
+                         stream, a);
+    });
   }
-  switch (table_chunks(a.E)) {
-    case 1: return launch_manage_tq<IDB, REMAP, 1>(a, stream);
-    case 2: return launch_manage_tq<IDB, REMAP, 2>(a, stream);
-    case 4: return launch_manage_tq<IDB, REMAP, 4>(a, stream);
-    default: return launch_manage_tq<IDB, REMAP, kTabRegs>(a, stream);
-  }
-}
-
-template <int TQ>
-int launch_prefetch_tq(const ManageArgs& a, hipStream_t stream) {
-  const dim3 grid(1), block(kWave);
-  if (a.S <= 64)
-    hipLaunchKernelGGL((prefetch_k<1, false, TQ>), grid, block, 0, stream, a);
-  else if (a.S <= 128)
-    hipLaunchKernelGGL((prefetch_k<2, false, TQ>), grid, block, 0, stream, a);
-  else if (a.S <= 256)
-    hipLaunchKernelGGL((prefetch_k<4, false, TQ>), grid, block, 0, stream, a);
-  else if (a.S <= 512)
-    hipLaunchKernelGGL((prefetch_k<8, false, TQ>), grid, block, 0, stream, a);
-  else
-    hipLaunchKernelGGL((prefetch_k<16, false, TQ>), grid, block, 0, stream, a);
   return (int)hipGetLastError();
 }
 
 int launch_prefetch(const ManageArgs& a, hipStream_t stream) {
   if (a.E > kLdsExperts) {
-    hipLaunchKernelGGL((prefetch_k<16, true, kTabRegs>), dim3(1), dim3(kWave), 0, stream, a);
-    return (int)hipGetLastError();
+    hipLaunchKernelGGL((prefetch_k<16, true>), dim3(1), dim3(16 * kWave), 0, stream, a);
+  } else {
+    with_waves(waves_for(a.E, a.S, a.mk), [&](auto w) {
+      hipLaunchKernelGGL((prefetch_k<w(), false>), dim3(1), dim3(w() * kWave), 0, stream, a);
+    });
   }
-  switch (table_chunks(a.E)) {
-    case 1: return launch_prefetch_tq<1>(a, stream);
-    case 2: return launch_prefetch_tq<2>(a, stream);
-    case 4: return launch_prefetch_tq<4>(a, stream);
-    default: return launch_prefetch_tq<kTabRegs>(a, stream);
-  }
-}
-
-// Both layers share E and S, so one variant serves the two workgroups.
-template <int IDB, int TQ>
-int launch_manage_prefetch_tq(const ManageArgs& a, const ManageArgs& p, hipStream_t stream) {
-  const dim3 grid(2), block(kWave);
-  if (a.S <= 64)
-    hipLaunchKernelGGL((manage_prefetch_k<1, false, IDB, TQ>), grid, block, 0, stream, a, p);
-  else if (a.S <= 128)
-    hipLaunchKernelGGL((manage_prefetch_k<2, false, IDB, TQ>), grid, block, 0, stream, a, p);
-  else if (a.S <= 256)
-    hipLaunchKernelGGL((manage_prefetch_k<4, false, IDB, TQ>), grid, block, 0, stream, a, p);
-  else if (a.S <= 512)
-    hipLaunchKernelGGL((manage_prefetch_k<8, false, IDB, TQ>), grid, block, 0, stream, a, p);
-  else
-    hipLaunchKernelGGL((manage_prefetch_k<16, false, IDB, TQ>), grid, block, 0, stream, a, p);
   return (int)hipGetLastError();
 }
 
+// Both layers share E and S, so one variant serves the two workgroups.
 template <int IDB>
 int launch_manage_prefetch(const ManageArgs& a, const ManageArgs& p, hipStream_t stream) {
   if (a.E > kLdsExperts) {
-    hipLaunchKernelGGL((manage_prefetch_k<16, true, IDB, kTabRegs>), dim3(2), dim3(kWave), 0,
+    hipLaunchKernelGGL((manage_prefetch_k<16, true, IDB>), dim3(2), dim3(16 * kWave), 0,
                        stream, a, p);
-    return (int)hipGetLastError();
+  } else {
+    with_waves(waves_for(a.E, a.S, a.mk > p.mk ? a.mk : p.mk), [&](auto w) {
+      hipLaunchKernelGGL((manage_prefetch_k<w(), false, IDB>), dim3(2), dim3(w() * kWave), 0,
+                         stream, a, p);
+    });
   }
-  switch (table_chunks(a.E)) {
-    case 1: return launch_manage_prefetch_tq<IDB, 1>(a, p, stream);
-    case 2: return launch_manage_prefetch_tq<IDB, 2>(a, p, stream);
-    case 4: return launch_manage_prefetch_tq<IDB, 4>(a, p, stream);
-    default: return launch_manage_prefetch_tq<IDB, kTabRegs>(a, p, stream);
-  }
-}
-
-template <int TQ>
-int launch_fused_tq(const ManageArgs& a, const AlignArgs& g, hipStream_t stream) {
-  const dim3 grid(1), block(kWave);
-  if (a.S <= 64)
-    hipLaunchKernelGGL((fused_k<1, TQ>), grid, block, 0, stream, a, g);
-  else if (a.S <= 128)
-    hipLaunchKernelGGL((fused_k<2, TQ>), grid, block, 0, stream, a, g);
-  else if (a.S <= 256)
-    hipLaunchKernelGGL((fused_k<4, TQ>), grid, block, 0, stream, a, g);
-  else if (a.S <= 512)
-    hipLaunchKernelGGL((fused_k<8, TQ>), grid, block, 0, stream, a, g);
-  else
-    hipLaunchKernelGGL((fused_k<16, TQ>), grid, block, 0, stream, a, g);
   return (int)hipGetLastError();
 }
 
 int launch_fused(const ManageArgs& a, const AlignArgs& g, hipStream_t stream) {
-  switch (table_chunks(a.E)) {
-    case 1: return launch_fused_tq<1>(a, g, stream);
-    case 2: return launch_fused_tq<2>(a, g, stream);
-    case 4: return launch_fused_tq<4>(a, g, stream);
-    default: return launch_fused_tq<kTabRegs>(a, g, stream);
+  if (a.mk <= kFusedIds) {
+    with_waves(waves_for(a.E, a.S, 4 * a.mk), [&](auto w) {
+      hipLaunchKernelGGL((fused_k<w()>), dim3(1), dim3(w() * kWave), 0, stream, a, g);
+    });
+    return (int)hipGetLastError();
   }
+  const int rc = launch_manage<4, false>(a, stream);
+  if (rc) return rc;
+  hipLaunchKernelGGL(align_k, dim3((a.mk - 1) / 1024 + 1), dim3(1024), 0, stream,
+                     static_cast<const int*>(a.ids), a.mk, a.E, a.S, a.table, g);
+  return (int)hipGetLastError();
 }
 
 ManageArgs make_args(const void* ids, int mk, int E, int S, int max_distinct, int max_inserts,

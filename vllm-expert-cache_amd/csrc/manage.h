@@ -1,25 +1,32 @@
-// expert_cache_manage on gfx950: one policy step of one layer's cache in ONE wavefront.
+// expert_cache_manage on gfx950: one policy step of one layer's cache in ONE workgroup.
 //
 // Behaviour follows kernels/expert_cache.hip:191-282 and tests/test_policy.py:83-132
 // (the step is restated in oracle/policy.c); the structure is this file's own:
 //
-//  * Every global load the step needs (step counter, ids, slot_expert, slot_stamp, the
-//    first 512 table entries) is issued up front, so the step costs one memory round trip
-//    plus the stores. There are no workgroup barriers: all cross-lane traffic is DPP,
-//    ballots, or LDS ordered by lgkmcnt waits.
-//  * Slots live in registers, CS per lane (slot s = lane + 64*c). The LDS holds the routed
-//    flags and the table (for E <= 4096) so that the remap can read the updated table
-//    without another trip to memory.
+//  * The workgroup has W waves, as many as give every expert and every slot a thread of its
+//    own (64 W >= E and S; above 1024 experts 16 waves walk the experts). What bounds the
+//    step is latency, and a large part of it is instruction fetch: a launch finds its code
+//    in no cache of the XCD it lands on. With one element a thread every phase is one short
+//    piece of straight code, whatever E and S.
+//  * Every global load the step needs (step counter, ids, slot_expert, slot_stamp, table) is
+//    issued up front, so the step costs one memory round trip plus the stores. Cross-lane
+//    traffic is DPP and ballots, cross-wave traffic LDS behind barriers that wait for LDS
+//    operations only.
+//  * The LDS holds the routed flags and the table so that the remap can read the updated
+//    table without another trip to memory.
 //  * Misses are enumerated in ascending expert id with ballot + popcount prefixes.
-//  * Victims are the nact smallest keys (stamp << 20 | slot) among the slots whose expert
-//    is not routed this step, assigned in ascending key order to the misses in ascending
-//    id order. Few inserts: repeated DPP wave-min (one 6-step DPP reduction per insert).
-//    Many inserts: a binary search on the key value finds the nact-th smallest key (each
-//    probe one ballot count per register chunk); the victims at or below it are ranked
-//    among themselves. Both give the same assignment (keys are unique, installing does not
-//    change any other slot's key or evictability).
-//  * A fused tail rewrites the caller's routing ids into slot ids against the updated table
-//    (vllm_expert_cache/cache.py:108-110 semantics, negative ids wrapping).
+//  * Victims are the nact smallest keys (stamp << 20 | slot) among the slots whose expert is
+//    not routed this step, assigned in ascending key order to the misses in ascending id
+//    order. They are found on 32-bit keys that order the same way (victim_key32): the first
+//    wave takes the minimum of all keys once per insert where inserts are few; otherwise
+//    every wave sorts its 64 keys in registers and the first wave merges the sorted lists
+//    down to the 64 smallest, or, for more victims than that, a key's rank is found by a
+//    binary search in each list. Stamps too far apart for 32 bits are ranked on the 64-bit
+//    keys by counting.
+//
+// Measured on MI355X, us for a graph of 48 launches, against a one-wave kernel that held up to
+// 16 slots and 8 experts a lane: 128 experts, 64 slots, 8 ids 111 -> 104; 256, 192, 128 ids,
+// 6.6 inserts a launch 246 -> 159; 512, 257, 50 ids, 2.6 inserts 274 -> 153.
 #pragma once
 #include <type_traits>
 
@@ -31,10 +38,9 @@ constexpr int kSlotBits = 20;
 constexpr int kSlotMask = (1 << kSlotBits) - 1;
 constexpr int kMaxSlots = 1024;
 constexpr int kMaxInserts = 1024;
-constexpr int kLdsExperts = 4096;   // flags + table fit in LDS up to this many experts
-constexpr int kIdRegs = 4;          // ids held in registers: mk <= 256
-constexpr int kTabRegs = 8;         // most table entries held per lane: E <= 512
+constexpr int kLdsExperts = 1024;   // flags + table are in LDS up to this many experts
 constexpr long long kKeyMax = 0x7FFFFFFFFFFFFFFFll;
+constexpr unsigned kKeyNone = 0xFFFFFFFFu;  // 32-bit key of a slot that cannot be evicted
 
 struct ManageArgs {
   const void* ids;
@@ -53,14 +59,18 @@ struct ManageArgs {
 
 // Experts above kLdsExperts (GLOBAL_E) keep their flags in the caller's `routed` buffer and
 // read the table from memory; the LDS arrays for them shrink to one element.
-template <bool GLOBAL_E>
+template <int W, bool GLOBAL_E>
 struct ManageLds {
-  alignas(16) unsigned char flag[GLOBAL_E ? 16 : kLdsExperts];  // cleared 16 bytes a lane
-  alignas(16) unsigned char hit[kMaxSlots];  // slot refreshed by a routed expert this step
-  int tab[GLOBAL_E ? 1 : kLdsExperts];
-  alignas(16) long long key[kMaxSlots + 8];  // select path: victim keys, INT64_MAX padded
-  int rank[kMaxSlots];             // select path: key order of each compacted victim
-  int mis[kMaxInserts];            // insert r -> missing expert
+  static constexpr int T = W * kWave;
+  alignas(16) unsigned char flag[GLOBAL_E ? 16 : T];  // expert routed this step
+  alignas(16) unsigned char hit[T];  // slot refreshed by a routed expert this step
+  int tab[GLOBAL_E ? 1 : T];
+  unsigned key[T];      // victim keys (sorted within each wave where every wave sorts)
+  int ins[T];           // slot -> insert it takes, or -1
+  int mis[T];           // insert r -> missing expert
+  long long key64[T];   // 64-bit victim keys, where the stamps need them
+  long long wmin[W];
+  int wsum[2][W], wev[W];
 };
 
 template <int IDB>
@@ -87,18 +97,38 @@ __device__ __forceinline__ void step_sync() {
     lds_sync();
 }
 
+__device__ __forceinline__ int wave_index() {
+  return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+}
+
 __device__ __forceinline__ long long victim_key(long long stamp, int slot) {
   return (long long)(((unsigned long long)stamp << kSlotBits) | (unsigned long long)slot);
 }
 
-// Which victim search is cheaper: a wave-min reduction plus its install per insert
-// (measured on gfx950: ~0.27 us per insert with one slot per lane, ~0.3-0.6 us with 2-8),
-// or the threshold select, whose cost hardly depends on the insert count (~1.3 us with one
-// slot per lane, ~2-3.6 us with 2-8). The crossovers are about 3 and 6 inserts.
-template <int CS>
-__device__ __forceinline__ bool use_argmin(int nact, int nev) {
-  (void)nev;
-  return nact <= (CS == 1 ? 3 : 6);
+// The 32-bit key of a stamp at or above `base` >= 1 (and below 2^43, where victim_key does
+// not overflow), in the order of victim_key: SB low bits of slot, above them 0 for stamp -1
+// (a pending prefetch), 1 for stamp 0 (an empty slot), then stamp - base + 2. `fits` is
+// false where the stamp has no such key.
+template <int SB>
+__device__ __forceinline__ unsigned victim_key32(long long stamp, long long base, int slot,
+                                                 bool& fits) {
+  constexpr unsigned long long kTop = (1ull << (32 - SB)) - 1;  // never a key: see kKeyNone
+  const unsigned long long rel =
+      stamp > 0 ? (unsigned long long)(stamp - base) + 2 : (unsigned long long)(stamp + 1);
+  fits = rel < kTop && stamp >= -1 && stamp < (1ll << 43) && (stamp <= 0 || stamp >= base);
+  return (unsigned)rel << SB | (unsigned)slot;
+}
+
+// Up to how many inserts the first wave finds the victims one by one. Measured on MI355X in
+// a graph of dependent launches that evict at every step (us a launch, one by one / sorted):
+// S = 48 of 64 experts 2.25 / 2.32 at 3 inserts, 2.37 / 2.33 at 5; S = 64 of 128 2.45 / 2.53
+// at 1, 2.58 / 2.55 at 3; S = 192 of 256 2.75 / 2.84 at 3, 3.07 / 2.87 at 6; S = 257 of 512
+// 3.21 / 3.34 at 4, 3.41 / 3.36 at 6; S = 900 of 1024 4.77 / 4.99 at 8, 5.09 / 4.93 at 10.
+// One by one costs 0.05-0.2 us more an insert, sorted stays level, so the line rises with
+// the number of lists to merge.
+template <int W>
+__device__ __forceinline__ int few_inserts(int S) {
+  return W == 1 ? 3 : 2 + S / 128;
 }
 
 __device__ __forceinline__ long long uniform_i64(long long v) {
@@ -108,13 +138,8 @@ __device__ __forceinline__ long long uniform_i64(long long v) {
   return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
-// Table chunks of 64 experts a lane holds in registers for E experts: the launch picks the
-// smallest of 1, 2, 4, 8 that covers E (8 also above 512 experts, which the general loops
-// handle), so small expert counts do not carry code for 512.
-constexpr int table_chunks(int E) { return E <= 64 ? 1 : E <= 128 ? 2 : E <= 256 ? 4 : 8; }
-
-// One policy step. On return, the updated table is in L.tab (or in memory for GLOBAL_E)
-// and idv holds ids[lane + 64k] (or -1 past mk). TQ table chunks are held in registers.
+// One policy step. On return, the updated table is in L.tab (or in memory for GLOBAL_E),
+// behind a sync that the caller makes, and idv holds ids[threadIdx.x] (or -1 past mk).
 //
 // PF makes it the prefetch step for predicted ids: the step counter is neither read nor
 // written, resident predicted experts keep their stamps, there is no ageing, and installs
@@ -127,462 +152,328 @@ constexpr int table_chunks(int E) { return E <= 64 ? 1 : E <= 128 ? 2 : E <= 256
 // whose expert is not routed is dropped -- the expert leaves the table and the slot is left
 // empty at stamp 0, so a prefetch copy still in flight may stop short. The reference never
 // holds a negative stamp, so on its states none of this runs.
-template <int CS, bool GLOBAL_E, int IDB, int TQ, bool PF = false>
-__device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<GLOBAL_E>& L,
-                                            long long (&idv)[kIdRegs]) {
+template <int W, bool GLOBAL_E, int IDB, bool PF = false>
+__device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GLOBAL_E>& L,
+                                            long long& idv) {
   static_assert(!PF || IDB == 4, "prefetch takes int32 ids");
-  const int lane = __lane_id();
+  static_assert(!GLOBAL_E || W == 16, "insert lists of 1024 experts");
+  constexpr int T = W * kWave;
+  constexpr int SB = W == 1 ? 6 : W == 2 ? 7 : W == 4 ? 8 : W == 8 ? 9 : 10;
+  const int tid = threadIdx.x, lane = __lane_id(), wave = wave_index();
   const int E = a.E, S = a.S, mk = a.mk;
+  const bool slot = tid < S;
 
   // ---- every independent load, issued together ---------------------------------------
   // Addresses are clamped into range instead of predicated, so no load waits behind a
-  // branch; lanes past the end substitute their sentinel after the loads return. The step
+  // branch; threads past the end substitute their sentinel after the loads return. The step
   // counter is a vector load: a scalar load would count in lgkmcnt, and every LDS fence
   // below would stall on it.
   long long st_v = 0;
   if constexpr (!PF)
     st_v = __hip_atomic_load(a.step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // No branch around the id loads either (a branch join would make the compiler wait for
-  // them before issuing the rest): with no ids, they read the 8-byte step counter (the
+  // No branch around the id load either (a branch join would make the compiler wait for
+  // it before issuing the rest): with no ids, it reads the 8-byte step counter (the
   // prefetch step: the first table entry) instead.
   using IdT = typename std::conditional<IDB == 8, long long, int>::type;
   const IdT* dummy = PF ? reinterpret_cast<const IdT*>(a.table)
                         : reinterpret_cast<const IdT*>(a.step);
   const IdT* ip = mk > 0 ? reinterpret_cast<const IdT*>(a.ids) : dummy;
-  const int last_id = mk > 0 ? mk - 1 : 0;
-  IdT raw[kIdRegs];
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k) raw[k] = ip[min(lane + k * kWave, last_id)];
-  int se[CS];
-  long long sp[CS];
-#pragma unroll
-  for (int c = 0; c < CS; ++c) {
-    const int s = min(lane + c * kWave, S - 1);
-    se[c] = a.slot_expert[s];
-    sp[c] = a.slot_stamp[s];
-  }
-  int tv[TQ];
-  if constexpr (!GLOBAL_E) {
-#pragma unroll
-    for (int u = 0; u < TQ; ++u) tv[u] = a.table[min(lane + u * kWave, E - 1)];
-  }
-  unsigned char* flag;
-  if constexpr (GLOBAL_E)
-    flag = a.routed;
-  else
-    flag = L.flag;
+  const IdT raw = ip[min(tid, max(mk - 1, 0))];
+  int se = a.slot_expert[min(tid, S - 1)];
+  long long sp = a.slot_stamp[min(tid, S - 1)];
+  int tv = -1;
+  if constexpr (!GLOBAL_E) tv = a.table[min(tid, E - 1)];
 
-  // clears: 16 bytes per lane per store (E <= 4096 and S <= 1024 stay inside the arrays)
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  // clears: four bytes a thread
+  unsigned char* flag;
   if constexpr (GLOBAL_E) {
-    for (int e = lane; e < E; e += kWave) flag[e] = 0;
+    flag = a.routed;
+    for (int e = tid; e < E; e += T) flag[e] = 0;
   } else {
-    for (int i = lane * 16; i < E; i += kWave * 16)
-      *reinterpret_cast<u32x4*>(&L.flag[i]) = u32x4{0, 0, 0, 0};
+    flag = L.flag;
+    if (tid < T / 4) reinterpret_cast<unsigned*>(L.flag)[tid] = 0;
   }
-  for (int i = lane * 16; i < S; i += kWave * 16)
-    *reinterpret_cast<u32x4*>(&L.hit[i]) = u32x4{0, 0, 0, 0};
+  if (tid < T / 4) reinterpret_cast<unsigned*>(L.hit)[tid] = 0;
   step_sync<GLOBAL_E>();
 
   // ---- routed flags (ids outside [0,E) are padding; int64 ids truncate like .to(int32))
-  // The sentinels for lanes past mk / S are applied only now, after the first fence, so
+  // The sentinels for threads past mk / S are applied only now, after the first fence, so
   // that fence does not wait for the loads.
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k)
-    idv[k] = (mk > 0 && lane + k * kWave < mk) ? (long long)raw[k] : -1;
-#pragma unroll
-  for (int c = 0; c < CS; ++c)
-    if (lane + c * kWave >= S) se[c] = -1;
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k) {
-    const int e = (int)idv[k];
+  idv = tid < mk ? (long long)raw : -1;
+  if (!slot) se = -1;
+  {
+    const int e = (int)idv;
     if (e >= 0 && e < E) flag[e] = 1;
   }
-  for (int i = lane + kIdRegs * kWave; i < mk; i += kWave) {
-    const int e = (int)load_id<IDB>(a.ids, i);
-    if (e >= 0 && e < E) flag[e] = 1;
+  for (unsigned i = tid + T; (int)i < mk; i += 4 * T) {
+    int e[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) e[k] = (int)ip[min(i + k * T, (unsigned)(mk - 1))];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (e[k] >= 0 && e[k] < E) flag[e[k]] = 1;
   }
-  if constexpr (!GLOBAL_E) {
-    // entries past E (below 512) are written too: nothing reads them
-#pragma unroll
-    for (int u = 0; u < TQ; ++u) L.tab[lane + u * kWave] = tv[u];
-    for (int base = TQ * kWave; base < E; base += kTabRegs * kWave) {
-      int tw[kTabRegs];
-#pragma unroll
-      for (int u = 0; u < kTabRegs; ++u) tw[u] = a.table[min(base + lane + u * kWave, E - 1)];
-#pragma unroll
-      for (int u = 0; u < kTabRegs; ++u) {
-        const int e = base + lane + u * kWave;
-        if (e < E) L.tab[e] = tw[u];
-      }
-    }
-  }
+  if constexpr (!GLOBAL_E) L.tab[tid] = tv;  // entries past E are written too: nothing reads them
   step_sync<GLOBAL_E>();
 
-  // ---- distinct count (the caller's `routed` is left holding the flags), then hits mark
-  // ---- their slot and misses enumerate in ascending expert id ------------------------
-  int cnt = 0, total = 0;
-  if (!GLOBAL_E && E <= TQ * kWave) {
-    // the whole table is in registers: one batch of flag reads, no table re-read; chunks
-    // past E are skipped on a uniform branch
-    const int nchunk = (E + kWave - 1) / kWave;
-    unsigned char fb[TQ];
-    bool fl[TQ];
-#pragma unroll
-    for (int u = 0; u < TQ; ++u) fb[u] = flag[min(lane + u * kWave, E - 1)];
-#pragma unroll
-    for (int u = 0; u < TQ; ++u) fl[u] = (fb[u] != 0) & (lane + u * kWave < E);
-#pragma unroll
-    for (int u = 0; u < TQ; ++u) {
-      if (u < nchunk) {
-        // lanes past E store routed[E-1]'s own flag there: no store needs a branch
-        a.routed[min(lane + u * kWave, E - 1)] = fb[u] != 0 ? 1 : 0;
-        cnt += __popcll(__ballot(fl[u]));
-      }
+  // ---- distinct count (the caller's `routed` is left holding the flags); hits mark their
+  // ---- slot; misses enumerate in ascending expert id ----------------------------------
+  const bool held = slot & (se >= 0) & (se < E);
+  const bool fx = held & (flag[held ? se : 0] != 0);  // the slot's expert is routed
+  int total = 0, distinct = 0;
+  if constexpr (!GLOBAL_E) {
+    const unsigned char fb = flag[tid];  // zero past E
+    if (tid < E) a.routed[tid] = fb;
+    const bool m = (fb != 0) & (tv < 0);
+    if (!PF && fb != 0 && tv >= 0 && tv < S) L.hit[tv] = 1;
+    const unsigned long long mask = __ballot(m);
+    // both counts in one word: neither exceeds 1024 over the workgroup
+    const int mine = (int)(__popcll(__ballot(fb != 0)) << 16 | __popcll(mask));
+    int before = 0, all = mine;
+    if constexpr (PF) {
+      // the prefetch step has no step counter to measure stamps from: their maximum serves
+      const long long top = wave_min_i64(~(slot ? sp : 0));
+      if (lane == 0) L.wmin[wave] = top;
     }
-    if (cnt > a.max_distinct) {  // wide step: read through, nothing else changes
-      if (lane == 0) {
-        if constexpr (!PF) a.step[0] = st_v + 1;
-        a.n_miss[0] = 0;
-      }
-      return;
+    if constexpr (W > 1) {
+      if (lane == 0) L.wsum[0][wave] = mine;
     }
-#pragma unroll
-    for (int u = 0; u < TQ; ++u) {
-      if (u < nchunk) {
-        const int e = lane + u * kWave;
-        const int t = tv[u];
-        if (!PF && fl[u] && t >= 0 && t < S) L.hit[t] = 1;
-        const bool m = fl[u] && t < 0;
-        const unsigned long long mask = __ballot(m);
-        const int j = total + __popcll(mask & lanes_below());
-        if (m && j < a.max_inserts) L.mis[j] = e;
-        total += __popcll(mask);
-      }
+    lds_sync();
+    if constexpr (W > 1) wave_sums<W>(L.wsum[0], wave, before, all);
+    distinct = all >> 16;
+    total = all & 0xFFFF;
+    const int j = (before & 0xFFFF) + __popcll(mask & lanes_below());
+    if (m && j < a.max_inserts && distinct <= a.max_distinct) {
+      L.mis[j] = tid;
+      a.miss[2 * j] = tid;
     }
   } else {
-    for (int base = 0; base < E; base += kWave) {
-      const int e = base + lane;
-      const bool f = e < E && flag[e];
-      if constexpr (!GLOBAL_E) {
-        if (e < E) a.routed[e] = f ? 1 : 0;
-      }
-      cnt += __popcll(__ballot(f));
-    }
-    if (cnt > a.max_distinct) {
-      if (lane == 0) {
-        if constexpr (!PF) a.step[0] = st_v + 1;
-        a.n_miss[0] = 0;
-      }
-      return;
-    }
-    for (int base = 0; base < E; base += kWave) {
-      const int e = base + lane;
-      const bool f = e < E && flag[e];
-      int t = -1;
-      if (f) {
-        if constexpr (GLOBAL_E)
-          t = a.table[e];
-        else
-          t = L.tab[e];
-      }
-      if (!PF && f && t >= 0 && t < S) L.hit[t] = 1;
-      const bool m = f && t < 0;
-      const unsigned long long mask = __ballot(m);
-      const int j = total + __popcll(mask & lanes_below());
-      if (m && j < a.max_inserts) L.mis[j] = e;
-      total += __popcll(mask);
-    }
-  }
-  const int nins = min(total, a.max_inserts);
-  lds_sync();
-
-  // ---- slot side: refreshed stamps, whether each slot's expert is routed, and pending
-  // ---- prefetch installs confirmed or dropped -----------------------------------------
-  const long long st = uniform_i64(st_v) + 1;
-  const bool lru = a.policy == 0;
-  const long long fresh = PF ? -1 : lru ? st : 1;
-  bool fx[CS];
-  // all flag reads first, with clamped indexes, so they are in flight together (a
-  // short-circuit test would put each read behind its own branch and wait)
-  unsigned char hv[CS], fv[CS];
-#pragma unroll
-  for (int c = 0; c < CS; ++c) {
-    hv[c] = L.hit[min(lane + c * kWave, S - 1)];
-    fv[c] = flag[min(max(se[c], 0), E - 1)];
-  }
-  int sign = 0;  // the OR of the stamps' high words: negative iff a stamp is
-#pragma unroll
-  for (int c = 0; c < CS; ++c) {
-    const int x = se[c];
-    fx[c] = (x >= 0) & (x < E) & (fv[c] != 0);
-    sign |= (int)((unsigned long long)sp[c] >> 32);
-  }
-  const bool ageing = !PF && !lru && nins > 0 && a.decay > 0 && (st % (long long)a.decay) == 0;
-  // Pending prefetch installs (negative stamps; none on the reference's states) are
-  // settled first, behind one wave-uniform branch, one slot per lane and iteration through
-  // LDS so the code stays small whatever the slots per lane. An unrouted one is dropped; a
-  // routed one is handed to the hit refresh below at the stamp that makes it end the step
-  // at an install's stamp: 0 (+1 = 1 under LFU; st under LRU), or 1 when this step ages
-  // (+1, halved = 1).
-  if (!PF && __ballot(sign < 0) != 0) {
-#pragma unroll
-    for (int c = 0; c < CS; ++c) {
-      const int s = lane + c * kWave;
-      if (s < S) {
-        L.key[s] = sp[c];
-        L.rank[s] = se[c];
-      }
+    int n = 0;
+    for (int e = tid; e < E; e += T) n += flag[e] != 0;
+    n = wave_incl_scan(n);
+    if (lane == kWave - 1) L.wsum[1][wave] = n;
+    if constexpr (PF) {
+      const long long top = wave_min_i64(~(slot ? sp : 0));
+      if (lane == 0) L.wmin[wave] = top;
     }
     lds_sync();
-#pragma unroll 1
-    for (int s = lane; s < S; s += kWave) {
-      const int x = L.rank[s];
-      if (L.key[s] < 0 && x >= 0 && x < E) {
-        if (flag[x]) {
-          L.key[s] = ageing ? 1 : 0;
-          L.hit[s] = 1;
-        } else {  // distinct slots hold distinct experts: no write conflicts
-          a.table[x] = -1;
-          a.map_cold[x] = x;
-          if constexpr (!GLOBAL_E) L.tab[x] = -1;
-          L.rank[s] = -1;
-          L.key[s] = 0;
-          if (nins == 0) {
-            a.slot_expert[s] = -1;
-            a.slot_stamp[s] = 0;
-          }
+    int before;
+    wave_sums<W>(L.wsum[1], wave, before, distinct);
+    lds_sync();
+    if (distinct <= a.max_distinct) {
+      int buf = 0;
+      for (int base = 0; base < E; base += T, buf ^= 1) {
+        const int e = base + tid;
+        const bool f = e < E && flag[e];
+        const int t = f ? a.table[e] : -1;
+        if (!PF && f && t >= 0 && t < S) L.hit[t] = 1;
+        const bool m = f && t < 0;
+        const unsigned long long mask = __ballot(m);
+        if (lane == 0) L.wsum[buf][wave] = __popcll(mask);
+        lds_sync();
+        int all;
+        wave_sums<W>(L.wsum[buf], wave, before, all);
+        const int j = total + before + __popcll(mask & lanes_below());
+        if (m && j < a.max_inserts) {
+          L.mis[j] = e;
+          a.miss[2 * j] = e;
         }
+        total += all;
       }
     }
-    lds_sync();
-#pragma unroll
-    for (int c = 0; c < CS; ++c) {
-      const int s = min(lane + c * kWave, S - 1);
-      sp[c] = L.key[s];
-      se[c] = lane + c * kWave < S ? L.rank[s] : -1;
-      hv[c] = L.hit[s];
-    }
   }
-#pragma unroll
-  for (int c = 0; c < CS; ++c) {
-    const int s = lane + c * kWave;
-    const bool hit = !PF && (s < S) & (hv[c] != 0);
-    if (hit) sp[c] = lru ? st : (long long)((unsigned long long)sp[c] + 1ull);
-    if (nins == 0 && hit) a.slot_stamp[s] = sp[c];
-  }
-  if (nins == 0) {  // no inserts: refreshed stamps only, no ageing
-    if (lane == 0) {
+  const long long st = uniform_i64(st_v) + 1;
+  if (distinct > a.max_distinct) {  // wide step: read through, nothing else changes
+    if (tid == 0) {
       if constexpr (!PF) a.step[0] = st;
       a.n_miss[0] = 0;
     }
     return;
   }
+  const int nins = min(total, a.max_inserts);
 
-  // LFU ageing on inserting steps where st % decay == 0
-  if (ageing) {
-#pragma unroll
-    for (int c = 0; c < CS; ++c) sp[c] >>= 1;
-  }
-
-  // ---- keys of the evictable slots (expert not routed this step) ---------------------
-  long long key[CS];
-  bool ev[CS];
-  int nev = 0;
-#pragma unroll
-  for (int c = 0; c < CS; ++c) {
-    const int s = lane + c * kWave;
-    ev[c] = s < S && !fx[c];
-    key[c] = victim_key(sp[c], s);
-    nev += __popcll(__ballot(ev[c]));
-  }
-  const int nact = min(nins, nev);
-
-  if (use_argmin<CS>(nact, nev)) {
-    // ---- few inserts: repeated wave-min, each insert installed as soon as it is found.
-    // The victim's old expert comes from its owner lane's register, the insert r-th miss
-    // from lane r's copy of the miss list.
-    const int my_mis = L.mis[min(lane, nins - 1)];
-    for (int r = 0; r < nact; ++r) {
-      long long m = kKeyMax;
-#pragma unroll
-      for (int c = 0; c < CS; ++c)
-        if (ev[c] && key[c] < m) m = key[c];
-      m = wave_min_i64(m);
-      const int sl = (int)(m & kSlotMask);
-      const int csl = sl >> 6, lsl = sl & (kWave - 1);
-      const int e = __builtin_amdgcn_readlane(my_mis, r);
-      int old = -1;
-#pragma unroll
-      for (int c = 0; c < CS; ++c)
-        if (c == csl) old = __builtin_amdgcn_readlane(se[c], lsl);
-#pragma unroll
-      for (int c = 0; c < CS; ++c)
-        if (c == csl && lane == lsl) {
-          ev[c] = false;
-          se[c] = e;
-          sp[c] = fresh;
-        }
-      if (lane == 0) {
-        if (old >= 0 && old < E) {
-          a.table[old] = -1;
-          a.map_cold[old] = old;
-          if constexpr (!GLOBAL_E) L.tab[old] = -1;
-        }
-        a.table[e] = sl;
-        a.map_cold[e] = -1;
-        a.miss[2 * r + 1] = sl;
-        if constexpr (!GLOBAL_E) L.tab[e] = sl;
-      }
-    }
-  } else {
-    // ---- many inserts: threshold select. With h = key >> 20 (the stamp bits), sigma is
-    // ---- the smallest h such that at least nact evictable keys have h <= sigma, found by
-    // ---- binary search with one ballot count per register chunk per probe. Every
-    // ---- evictable key below bucket sigma is a victim; the rest of the nact come from
-    // ---- bucket sigma in slot order (= key order within a bucket). Each lane then installs
-    // ---- its own victims from registers (distinct slots, distinct experts, disjoint table
-    // ---- entries, so the installs need no ordering among themselves).
-    long long kmin = kKeyMax, nmax = kKeyMax;  // smallest key, and ~largest key
-#pragma unroll
-    for (int c = 0; c < CS; ++c) {
-      if (ev[c] && key[c] < kmin) kmin = key[c];
-      if (ev[c] && ~key[c] < nmax) nmax = ~key[c];
-    }
-    const long long hmin = wave_min_i64(kmin) >> kSlotBits;
-    const long long hmax = (~wave_min_i64(nmax)) >> kSlotBits;
-    long long sigma;
-    if ((unsigned long long)(hmax - hmin) < (1ull << 31)) {
-      // stamp spreads below 2^31: 32-bit compares on h - hmin (non-evictable: all ones)
-      unsigned rel[CS];
-#pragma unroll
-      for (int c = 0; c < CS; ++c)
-        rel[c] = ev[c] ? (unsigned)((key[c] >> kSlotBits) - hmin) : 0xFFFFFFFFu;
-      unsigned lo = 0, hi = (unsigned)(hmax - hmin);
-      while (lo < hi) {
-        const unsigned mid = (lo + hi) >> 1;
-        int n = 0;
-#pragma unroll
-        for (int c = 0; c < CS; ++c) n += __popcll(__ballot(rel[c] <= mid));
-        if (n >= nact)
-          hi = mid;
-        else
-          lo = mid + 1;
-      }
-      sigma = hmin + (long long)lo;
+  // ---- slot side: pending prefetch installs confirmed or dropped, refreshed stamps -------
+  const bool lru = a.policy == 0;
+  const long long fresh = PF ? -1 : lru ? st : 1;
+  const bool ageing = !PF && !lru && nins > 0 && a.decay > 0 && (st % (long long)a.decay) == 0;
+  bool hit = !PF && slot && L.hit[tid] != 0;
+  bool moved = false;  // slot_expert[tid] changes
+  bool aged = false;   // slot_stamp[tid] changes
+  if (!PF && held && sp < 0) {
+    // A routed one is handed to the hit refresh below at the stamp that makes it end the
+    // step at an install's stamp: 0 (+1 = 1 under LFU; st under LRU), or 1 when this step
+    // ages (+1, halved = 1). Distinct slots hold distinct experts: no write conflicts.
+    if (fx) {
+      sp = ageing ? 1 : 0;
+      hit = true;
     } else {
-      long long lo = hmin, hi = hmax;
-      while (lo < hi) {
-        const long long mid = lo + ((hi - lo) >> 1);
-        int n = 0;
-#pragma unroll
-        for (int c = 0; c < CS; ++c) n += __popcll(__ballot(ev[c] && (key[c] >> kSlotBits) <= mid));
-        if (n >= nact)
-          hi = mid;
-        else
-          lo = mid + 1;
-      }
-      sigma = lo;
+      a.table[se] = -1;
+      a.map_cold[se] = se;
+      if constexpr (!GLOBAL_E) L.tab[se] = -1;
+      se = -1;
+      sp = 0;
+      moved = aged = true;
+    }
+  }
+  if (hit) {
+    sp = lru ? st : (long long)((unsigned long long)sp + 1ull);
+    aged = true;
+  }
+  int nact = 0;
+  if (nins > 0) {
+    if (ageing) {  // LFU ageing on inserting steps where st % decay == 0
+      sp >>= 1;
+      aged = true;
     }
 
-    // victims: below bucket sigma, or in it among the first `need` by slot
-    bool below[CS], inb[CS];
-    int nbelow = 0;
-#pragma unroll
-    for (int c = 0; c < CS; ++c) {
-      const long long h = key[c] >> kSlotBits;
-      below[c] = ev[c] && h < sigma;
-      inb[c] = ev[c] && h == sigma;
-      nbelow += __popcll(__ballot(below[c]));
+    // ---- keys of the evictable slots (expert not routed this step) -------------------
+    const bool ev = slot & !fx;
+    long long base = 1;
+    if constexpr (PF) {
+      long long top = kKeyMax;
+      for (int w = 0; w < W; ++w) top = min(top, L.wmin[w]);
+      base = max(1ll, ~top - ((1ll << (32 - SB)) - 8));
+    } else {
+      if (lru) base = max(1ll, st - ((1ll << (32 - SB)) - 8));
     }
-    const int need = nact - nbelow;
-    int pos[CS];  // insert index of each victim, or -1
-    int seen_b = 0, seen_in = 0;
-#pragma unroll
-    for (int c = 0; c < CS; ++c) {
-      const unsigned long long mb = __ballot(below[c]), mi = __ballot(inb[c]);
-      const int rb = seen_b + __popcll(mb & lanes_below());
-      const int ri = seen_in + __popcll(mi & lanes_below());
-      pos[c] = inb[c] && ri < need ? nbelow + ri : -1;
-      if (below[c]) {
-        L.key[rb] = key[c];
-        pos[c] = rb;  // compaction index until ranked
-      }
-      seen_b += __popcll(mb);
-      seen_in += __popcll(mi);
-    }
-    if (nbelow > 0) {
-      // victims below the bucket take inserts 0..nbelow-1 in key order: rank each among
-      // them (every lane reads the same keys, an LDS broadcast, 8 per batch)
-      const int n8 = (nbelow + 7) & ~7;
-      if (lane < n8 - nbelow) L.key[nbelow + lane] = kKeyMax;
+    bool fits;
+    unsigned key = victim_key32<SB>(sp, base, tid, fits);
+    if (!ev) key = kKeyNone;
+    const int nev_wave = (int)__popcll(__ballot(ev)) | (__ballot(ev & !fits) ? 1 << 16 : 0);
+    int nev = nev_wave;
+    const bool few = nins <= few_inserts<W>(S);
+    int r = -1;  // insert this thread's slot takes
+    if constexpr (W > 1) {
+      const unsigned sorted = few ? key : wave_sort(key);
+      L.key[tid] = sorted;
+      L.ins[tid] = -1;
+      if (lane == 0) L.wev[wave] = nev_wave;
       lds_sync();
-      typedef long long i64x2 __attribute__((ext_vector_type(2)));
-      const i64x2* kp = reinterpret_cast<const i64x2*>(L.key);
-      for (int j0 = 0; j0 < nbelow; j0 += kWave) {
-        const int j = j0 + lane;
-        const long long kj = L.key[min(j, n8 - 1)];
+      int before;
+      wave_sums<W>(L.wev, wave, before, nev);
+      nact = min(nins, nev & 0xFFFF);
+      if (nev <= 0xFFFF && nact <= kWave) {
+        if (wave == 0) {
+          unsigned v = sorted;  // to become, in lane i, the i-th smallest key
+          if (few) {
+            unsigned k[W];
+#pragma unroll
+            for (int c = 0; c < W; ++c)
+              k[c] = c * kWave < S ? L.key[c * kWave + lane] : kKeyNone;
+#pragma unroll 1
+            for (int i = 0; i < nact; ++i) {
+              unsigned m = k[0];
+#pragma unroll
+              for (int c = 1; c < W; ++c) m = min(m, k[c]);
+              m = wave_min_u32(m);
+              if (lane == i) v = m;
+#pragma unroll
+              for (int c = 0; c < W; ++c)
+                if (k[c] == m) k[c] = kKeyNone;
+            }
+          } else {
+#pragma unroll 1
+            for (int c = kWave; c < S; c += kWave)
+              v = wave_merge_low(v, L.key[c + kWave - 1 - lane]);
+          }
+          if (lane < nact) L.ins[v & (T - 1)] = lane;
+        }
+        lds_sync();
+        r = L.ins[tid];
+      } else if (nev <= 0xFFFF) {
+        // more victims than lanes: rank of this thread's sorted key, the keys below it in
+        // every wave's sorted list (in its own, its lane), four lists searched at a time
+        if (sorted != kKeyNone) {
+          int rank = 0;
+          const int lists = (S + kWave - 1) / kWave;
+#pragma unroll 1
+          for (int w0 = 0; w0 < lists; w0 += 4) {
+            int p[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int step = 32; step > 0; step >>= 1) {
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                if (q < W && L.key[min(w0 + q, W - 1) * kWave + p[q] + step - 1] < sorted)
+                  p[q] += step;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              if (q < W && w0 + q < lists)
+                rank += p[q] + (L.key[(w0 + q) * kWave + p[q]] < sorted ? 1 : 0);
+            }
+          }
+          if (rank < nact) L.ins[sorted & (T - 1)] = rank;
+        }
+        // the slots of a wave's keys are its own threads': ordered within the wave
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        r = L.ins[tid];
+      }
+    } else {
+      nact = min(nins, nev & 0xFFFF);
+      if (nev <= 0xFFFF) {
+        if (few) {
+#pragma unroll 1
+          for (int i = 0; i < nact; ++i) {
+            const unsigned m = wave_min_u32(key);
+            if (key == m) {
+              r = i;
+              key = kKeyNone;
+            }
+          }
+        } else {
+          const unsigned sorted = wave_sort(key);
+          L.ins[tid] = -1;
+          if (lane < nact && sorted != kKeyNone) L.ins[sorted & (T - 1)] = lane;
+          lds_sync();
+          r = L.ins[tid];
+        }
+      }
+    }
+    if (nev > 0xFFFF) {
+      // stamps too far apart for 32-bit keys: rank by counting on the 64-bit ones
+      const long long k64 = ev ? victim_key(sp, tid) : kKeyMax;
+      L.key64[tid] = k64;
+      lds_sync();
+      if (ev) {
         int rank = 0;
-        for (int i = 0; i < n8; i += 8) {
-          const i64x2 k01 = kp[i / 2], k23 = kp[i / 2 + 1], k45 = kp[i / 2 + 2],
-                      k67 = kp[i / 2 + 3];
-          rank += (k01.x < kj) + (k01.y < kj) + (k23.x < kj) + (k23.y < kj) + (k45.x < kj) +
-                  (k45.y < kj) + (k67.x < kj) + (k67.y < kj);
-        }
-        if (j < nbelow) L.rank[j] = rank;
-      }
-      lds_sync();
-#pragma unroll
-      for (int c = 0; c < CS; ++c)
-        if (below[c]) pos[c] = L.rank[pos[c]];
-    }
-
-    // installs, each by the lane holding the victim slot
-    int ne[CS];
-#pragma unroll
-    for (int c = 0; c < CS; ++c) ne[c] = L.mis[max(pos[c], 0)];
-#pragma unroll
-    for (int c = 0; c < CS; ++c) {
-      if (pos[c] >= 0) {
-        const int s = lane + c * kWave;
-        const int old = se[c], e = ne[c];
-        if (old >= 0 && old < E) {
-          a.table[old] = -1;
-          a.map_cold[old] = old;
-          if constexpr (!GLOBAL_E) L.tab[old] = -1;
-        }
-        a.table[e] = s;
-        a.map_cold[e] = -1;
-        a.miss[2 * pos[c] + 1] = s;
-        if constexpr (!GLOBAL_E) L.tab[e] = s;
-        se[c] = e;
-        sp[c] = fresh;
+#pragma unroll 4
+        for (int i = 0; i < S; ++i) rank += L.key64[i] < k64 ? 1 : 0;
+        if (rank < nact) r = rank;
       }
     }
-  }
-  step_sync<GLOBAL_E>();
 
-  // the caller's miss list gets every counted miss id (miss[2j], j < nins), also past nact
-  for (int j = lane; j < nins; j += kWave) a.miss[2 * j] = L.mis[j];
-#pragma unroll
-  for (int c = 0; c < CS; ++c) {
-    const int s = lane + c * kWave;
-    if (s < S) {
-      a.slot_expert[s] = se[c];
-      a.slot_stamp[s] = sp[c];
+    // ---- installs, each by the thread of the victim slot: distinct slots, distinct experts,
+    // ---- disjoint table entries, so they need no ordering among themselves ---------------
+    if constexpr (W == 1) lds_sync();  // L.mis, in the paths above that made no sync
+    if (r >= 0) {
+      const int e = L.mis[r];
+      if (se >= 0 && se < E) {
+        a.table[se] = -1;
+        a.map_cold[se] = se;
+        if constexpr (!GLOBAL_E) L.tab[se] = -1;
+      }
+      a.table[e] = tid;
+      a.map_cold[e] = -1;
+      a.miss[2 * r + 1] = tid;
+      if constexpr (!GLOBAL_E) L.tab[e] = tid;
+      se = e;
+      sp = fresh;
+      moved = aged = true;
     }
   }
-  if (lane == 0) {
+  if (slot && aged) a.slot_stamp[tid] = sp;
+  if (slot && moved) a.slot_expert[tid] = se;
+  if (tid == 0) {
     if constexpr (!PF) a.step[0] = st;
     a.n_miss[0] = nact;
   }
 }
 
 // out[i] = table[ids[i]] against the updated table, negative ids wrapping.
-template <bool GLOBAL_E, int IDB>
-__device__ __forceinline__ void remap_tail(const ManageArgs& a, const ManageLds<GLOBAL_E>& L,
-                                           const long long (&idv)[kIdRegs]) {
-  const int lane = __lane_id();
+template <int W, bool GLOBAL_E, int IDB>
+__device__ __forceinline__ void remap_tail(const ManageArgs& a,
+                                           const ManageLds<W, GLOBAL_E>& L, long long idv) {
+  const int tid = threadIdx.x;
   const int E = a.E, mk = a.mk;
   auto lookup = [&](long long v) -> int {
     if (v < 0) v += E;
@@ -592,12 +483,8 @@ __device__ __forceinline__ void remap_tail(const ManageArgs& a, const ManageLds<
     else
       return L.tab[v];
   };
-#pragma unroll
-  for (int k = 0; k < kIdRegs; ++k) {
-    const int i = lane + k * kWave;
-    if (i < mk) store_id<IDB>(a.out, i, lookup(idv[k]));
-  }
-  for (int i = lane + kIdRegs * kWave; i < mk; i += kWave)
+  if (tid < mk) store_id<IDB>(a.out, tid, lookup(idv));
+  for (int i = tid + W * kWave; i < mk; i += W * kWave)
     store_id<IDB>(a.out, i, lookup(load_id<IDB>(a.ids, i)));
 }
 
@@ -610,45 +497,43 @@ __device__ __forceinline__ void args_in_sgprs(const ManageArgs& a) {
                "s"(a.max_inserts), "s"(a.policy), "s"(a.decay));
 }
 
-template <int CS, bool GLOBAL_E, int IDB, bool REMAP, int TQ>
-__global__ __launch_bounds__(kWave) void manage_k(ManageArgs a) {
-  __shared__ ManageLds<GLOBAL_E> L;
+template <int W, bool GLOBAL_E, int IDB, bool REMAP>
+__global__ __launch_bounds__(W* kWave) void manage_k(ManageArgs a) {
+  __shared__ ManageLds<W, GLOBAL_E> L;
   args_in_sgprs(a);
-  long long idv[kIdRegs];
-  manage_step<CS, GLOBAL_E, IDB, TQ>(a, L, idv);
+  long long idv;
+  manage_step<W, GLOBAL_E, IDB>(a, L, idv);
   if constexpr (REMAP) {
-    if constexpr (GLOBAL_E) mem_sync();
-    else lds_sync();
-    remap_tail<GLOBAL_E, IDB>(a, L, idv);
+    step_sync<GLOBAL_E>();
+    remap_tail<W, GLOBAL_E, IDB>(a, L, idv);
   }
 }
 
 // The prefetch step (manage_step with PF) for int32 predicted ids.
-template <int CS, bool GLOBAL_E, int TQ>
-__global__ __launch_bounds__(kWave) void prefetch_k(ManageArgs a) {
-  __shared__ ManageLds<GLOBAL_E> L;
+template <int W, bool GLOBAL_E>
+__global__ __launch_bounds__(W* kWave) void prefetch_k(ManageArgs a) {
+  __shared__ ManageLds<W, GLOBAL_E> L;
   args_in_sgprs(a);
-  long long idv[kIdRegs];
-  manage_step<CS, GLOBAL_E, 4, TQ, true>(a, L, idv);
+  long long idv;
+  manage_step<W, GLOBAL_E, 4, true>(a, L, idv);
 }
 
 // Two workgroups, two layers: workgroup 0 runs layer a's policy step and remap (manage_k
 // with REMAP), workgroup 1 the prefetch step of another layer p (prefetch_k). The host
 // rejects states that share arrays, so the workgroups touch disjoint memory and need no
 // ordering between them; the pair occupies one node of the stream instead of two.
-template <int CS, bool GLOBAL_E, int IDB, int TQ>
-__global__ __launch_bounds__(kWave) void manage_prefetch_k(ManageArgs a, ManageArgs p) {
-  __shared__ ManageLds<GLOBAL_E> L;
-  long long idv[kIdRegs];
+template <int W, bool GLOBAL_E, int IDB>
+__global__ __launch_bounds__(W* kWave) void manage_prefetch_k(ManageArgs a, ManageArgs p) {
+  __shared__ ManageLds<W, GLOBAL_E> L;
+  long long idv;
   if (blockIdx.x == 0) {
     args_in_sgprs(a);
-    manage_step<CS, GLOBAL_E, IDB, TQ>(a, L, idv);
-    if constexpr (GLOBAL_E) mem_sync();
-    else lds_sync();
-    remap_tail<GLOBAL_E, IDB>(a, L, idv);
+    manage_step<W, GLOBAL_E, IDB>(a, L, idv);
+    step_sync<GLOBAL_E>();
+    remap_tail<W, GLOBAL_E, IDB>(a, L, idv);
   } else {
     args_in_sgprs(p);
-    manage_step<CS, GLOBAL_E, 4, TQ, true>(p, L, idv);
+    manage_step<W, GLOBAL_E, 4, true>(p, L, idv);
   }
 }
 

@@ -1,9 +1,5 @@
-// Wave64 primitives for gfx950 (CDNA4): DPP reductions/scans and LDS-only syncs.
-//
-// Every kernel in this library that uses them runs as ONE wavefront per workgroup, so a
-// "barrier" is only an ordering point for LDS traffic between lanes of that wave: the
-// compiler drops s_barrier for a 64-lane workgroup and the local-address-space fence
-// waits for LDS operations (lgkmcnt) only, leaving global loads in flight across it.
+// Wave64 primitives for gfx950 (CDNA4): DPP reductions/scans, a 64-lane sort, lane matching,
+// and workgroup syncs.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -12,15 +8,17 @@ namespace ec {
 
 constexpr int kWave = 64;
 
-// Orders LDS accesses of the wave before/after this point.
+// Orders the workgroup's LDS accesses before/after this point. The local-address-space
+// fences wait for LDS operations (lgkmcnt) only, so global loads and stores stay in flight
+// across it; for a workgroup of one wave the compiler drops the s_barrier.
 __device__ __forceinline__ void lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Orders LDS and global accesses of the wave before/after this point, and waits until the
-// wave's outstanding memory operations have completed.
+// Orders the workgroup's LDS and global accesses before/after this point, and waits until
+// its outstanding memory operations have completed.
 __device__ __forceinline__ void mem_sync() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
@@ -76,8 +74,132 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   return v;
 }
 
-__device__ __forceinline__ int wave_lane_value(int v, int lane) {
-  return __builtin_amdgcn_readlane(v, lane);
+// Minimum of `v` over all 64 lanes, returned to every lane (all lanes must be active).
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ unsigned dpp_umin_step(unsigned v) {
+  const unsigned o =
+      (unsigned)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, CTRL, ROWMASK, 0xF, false);
+  return o < v ? o : v;
+}
+
+__device__ __forceinline__ unsigned wave_min_u32(unsigned v) {
+  v = dpp_umin_step<0x111, 0xF>(v);
+  v = dpp_umin_step<0x112, 0xF>(v);
+  v = dpp_umin_step<0x114, 0xF>(v);
+  v = dpp_umin_step<0x118, 0xF>(v);
+  v = dpp_umin_step<0x142, 0xA>(v);
+  v = dpp_umin_step<0x143, 0xC>(v);
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The value of lane (own lane xor X). Rows of 16 lanes and quads are permuted by DPP, halves
+// of the wave by the permlane swaps (both operands `v`: the first result then holds the even
+// row / low half of each pair, the second the odd row / high half).
+template <int X>
+__device__ __forceinline__ unsigned lane_xor(unsigned v) {
+  static_assert(X == 1 || X == 2 || X == 3 || X == 4 || X == 7 || X == 8 || X == 15 ||
+                X == 16 || X == 31 || X == 32 || X == 63);
+  if constexpr (X == 1) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);
+  if constexpr (X == 2) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);
+  if constexpr (X == 3) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x1B, 0xF, 0xF, true);
+  if constexpr (X == 7) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);
+  if constexpr (X == 8) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);
+  if constexpr (X == 15) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true);
+  if constexpr (X == 4) return lane_xor<3>(lane_xor<7>(v));
+  if constexpr (X == 31) return lane_xor<16>(lane_xor<15>(v));
+  if constexpr (X == 63) return lane_xor<32>(lane_xor<31>(v));
+  if constexpr (X == 16) {
+    const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (__lane_id() & 16) ? p[0] : p[1];
+  }
+  if constexpr (X == 32) {
+    const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (__lane_id() & 32) ? p[0] : p[1];
+  }
+}
+
+// One compare-exchange of every lane with lane xor X: the lane with bit B set keeps the
+// larger value.
+template <int X, int B>
+__device__ __forceinline__ unsigned sort_step(unsigned v) {
+  const unsigned o = lane_xor<X>(v);
+  return (__lane_id() & B) ? max(v, o) : min(v, o);
+}
+
+// `v` sorted ascending over the 64 lanes: 21 compare-exchanges in registers. Each merge
+// starts with a mirrored exchange, so all of them run in ascending order.
+__device__ __forceinline__ unsigned wave_sort(unsigned v) {
+  v = sort_step<1, 1>(v);
+  v = sort_step<3, 2>(v);
+  v = sort_step<1, 1>(v);
+  v = sort_step<7, 4>(v);
+  v = sort_step<2, 2>(v);
+  v = sort_step<1, 1>(v);
+  v = sort_step<15, 8>(v);
+  v = sort_step<4, 4>(v);
+  v = sort_step<2, 2>(v);
+  v = sort_step<1, 1>(v);
+  v = sort_step<31, 16>(v);
+  v = sort_step<8, 8>(v);
+  v = sort_step<4, 4>(v);
+  v = sort_step<2, 2>(v);
+  v = sort_step<1, 1>(v);
+  v = sort_step<63, 32>(v);
+  v = sort_step<16, 16>(v);
+  v = sort_step<8, 8>(v);
+  v = sort_step<4, 4>(v);
+  v = sort_step<2, 2>(v);
+  v = sort_step<1, 1>(v);
+  return v;
+}
+
+// The 64 smallest of two sorted lists of 64, sorted: `v` ascending over the lanes, `down`
+// the other list descending. Their lane-wise minimum is those 64 as a bitonic sequence.
+__device__ __forceinline__ unsigned wave_merge_low(unsigned v, unsigned down) {
+  v = min(v, down);
+  v = sort_step<32, 32>(v);
+  v = sort_step<16, 16>(v);
+  v = sort_step<8, 8>(v);
+  v = sort_step<4, 4>(v);
+  v = sort_step<2, 2>(v);
+  v = sort_step<1, 1>(v);
+  return v;
+}
+
+// For a lane with v >= 0, the lanes whose `v` equals its own, compared on the low `bits`
+// bits (all lanes must be active). One ballot per bit: needs no LDS, and no order among the
+// lanes is assumed.
+__device__ __forceinline__ unsigned long long wave_match(int v, int bits) {
+  unsigned long long m = __ballot(v >= 0);
+#pragma unroll 1
+  for (int b = 0; b < bits; b += 4) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int bit = (v >> (b + k)) & 1;
+      m &= __ballot(bit) ^ ((unsigned long long)(long long)(bit - 1));
+    }
+  }
+  return m;
+}
+
+// Sums over the waves of a workgroup, from one word per wave in LDS (W <= 16): the words of
+// the waves before this one, and of all waves. Wave-uniform.
+template <int W>
+__device__ __forceinline__ void wave_sums(const int* word, int wave, int& before, int& all) {
+  if constexpr (W == 1) {
+    before = 0;
+    all = __builtin_amdgcn_readfirstlane(word[0]);
+  } else {
+    const int lane = __lane_id();
+    int v = word[min(lane, W - 1)];
+    v = dpp_add_step<0x111, 0xF>(v);
+    if constexpr (W > 2) v = dpp_add_step<0x112, 0xF>(v);
+    if constexpr (W > 4) v = dpp_add_step<0x114, 0xF>(v);
+    if constexpr (W > 8) v = dpp_add_step<0x118, 0xF>(v);
+    all = __builtin_amdgcn_readlane(v, W - 1);
+    const int prev = __builtin_amdgcn_readlane(v, max(wave - 1, 0));
+    before = wave > 0 ? prev : 0;
+  }
 }
 
 }  // namespace ec
