@@ -11,12 +11,11 @@
 // An id's rank is found without a pass over earlier ids: its lane's rank among the lanes of
 // its wave with the same bucket (wave_match), plus the counts of the earlier waves, which
 // each wave leaves in its own row of a small count matrix in LDS, plus, where several
-// workgroups share the ids, the count of the workgroup's earlier ids. No output position is
-// written twice (an id, its bucket's padding, or the default past the padded total), so
-// nothing is staged and no store is waited for.
+// workgroups share the ids, the count of the workgroup's earlier ids.
 //
 //  * fused_k, up to kFusedIds ids: the policy step and both alignments in one workgroup,
-//    one id, one expert and one slot a thread.
+//    one id, one expert and one slot a thread. Up to 64 ids are placed by one wave that
+//    sorts them in registers.
 //  * align_k, more ids: a workgroup per 1024 ids, after a launch of the policy step alone.
 //    Each workgroup counts the ids before and after its own itself (they come from the L2),
 //    which costs less than the node or the cross-XCD handoff that sharing the counts would.
@@ -34,6 +33,8 @@ constexpr int kFusedIds = 1024;  // most ids of the one-workgroup kernel: one a 
 
 struct AlignArgs {
   int bs, L, NB;
+  unsigned div_mul;  // x / bs = x * div_mul >> div_shift for 0 <= x < 2^31
+  int div_shift;
   int* sorted_hot;
   int* eids_hot;
   int* npad_hot;
@@ -64,16 +65,27 @@ __device__ __forceinline__ int align_key(int e, int E, int S, const int* tab) {
   return ((unsigned)s < (unsigned)S) ? s : S + e;
 }
 
-// x / bs for the wave-uniform block size: a shift for powers of two (vLLM's block sizes).
+// The multiplier and shift of the division by bs: with l = ceil(log2 bs), the multiplier is
+// 2^(31 + l) / bs rounded up (below 2^32), and the excess, below 1 / bs over x < 2^31, never
+// reaches the next quotient.
+inline void set_block_size(AlignArgs& g, int bs) {
+  int l = 0;
+  while ((1ll << l) < bs) ++l;
+  g.bs = bs;
+  g.div_shift = 31 + l;
+  g.div_mul = (unsigned)((((unsigned __int128)1 << g.div_shift) + bs - 1) / bs);
+}
+
 struct BlockDiv {
   int bs, shift;
-  __device__ __forceinline__ explicit BlockDiv(int b)
-      : bs(b), shift((b & (b - 1)) == 0 ? __builtin_ctz((unsigned)b) : -1) {}
-  __device__ __forceinline__ int div(int x) const { return shift >= 0 ? x >> shift : x / bs; }
+  unsigned mul;
+  __device__ __forceinline__ explicit BlockDiv(const AlignArgs& g)
+      : bs(g.bs), shift(g.div_shift), mul(g.div_mul) {}
+  __device__ __forceinline__ int div(int x) const {
+    return (int)((unsigned long long)(unsigned)x * mul >> shift);
+  }
   __device__ __forceinline__ int pad(int x) const { return div(x + bs - 1) * bs; }
 };
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // dst[from, to) = v over `n` threads of which this is number `me`; 16-byte stores when dst is
 // 16-byte aligned.
@@ -103,8 +115,9 @@ __device__ __forceinline__ void align_clear(AlignLds<W>& A, int waves, int bucke
 // Places id `i` of bucket `kk` (-1: none) for every thread of the workgroup, whose ids are
 // consecutive and lie in its first `waves` waves. The count matrix is clear. With PART the
 // workgroup holds only some of the ids: on entry A.start and A.end hold, per bucket, the
-// counts of the ids before and after its own. On return A.end and, per bucket, A.start are
-// positions as declared (behind the sync made here).
+// counts of the ids before and after its own; on return A.end and, per bucket, A.start are
+// positions as declared (behind the sync made here). Without it, the blocks' expert ids are
+// written too.
 template <int W, bool PART>
 __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<W>& A, int E,
                                                    int S, BlockDiv d, int kk, int i,
@@ -121,23 +134,19 @@ __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<
   // thread b: slot bucket b and expert bucket S + b
   int n[2] = {0, 0}, before[2] = {0, 0};
   const int size[2] = {S, E};
+  constexpr int kRows = W < 8 ? W : 8;  // rows read together
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int b = tid + (h ? S : 0);
     if (tid < size[h]) {
-      if (waves == 1) {
-        n[h] = A.cnt[0][b];
-        A.cnt[0][b] = 0;
-      } else {
-        for (int w0 = 0; w0 < waves; w0 += 4) {
-          int c[4];
+      for (int w0 = 0; w0 < waves; w0 += kRows) {
+        int c[kRows];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) c[q] = w0 + q < waves ? A.cnt[min(w0 + q, W - 1)][b] : 0;
+        for (int q = 0; q < kRows; ++q) c[q] = A.cnt[w0 + q][b];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            if (w0 + q < waves) A.cnt[min(w0 + q, W - 1)][b] = (unsigned short)n[h];
-            n[h] += c[q];
-          }
+        for (int q = 0; q < kRows; ++q) {
+          A.cnt[w0 + q][b] = (unsigned short)n[h];
+          if (w0 + q < waves) n[h] += c[q];  // the rows past the ids' are not clear
         }
       }
       if constexpr (PART) {
@@ -172,10 +181,19 @@ __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<
     if (tid < size[h]) {
       const int b = tid + (h ? S : 0);
       A.start[b] = first[h] + before[h];
-      A.end[b] = first[h] + n[h];
+      if constexpr (PART) A.end[b] = first[h] + n[h];
     }
   }
   lds_sync();
+  if constexpr (!PART) {
+    // thread b names the blocks of its two buckets
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int* eids = h ? g.eids_cold : g.eids_hot;
+      const int q1 = min(d.div(first[h] + padded[h]), g.NB);
+      for (int q = d.div(first[h]); q < q1; ++q) eids[q] = tid;
+    }
+  }
   if (kk >= 0) {
     const int pos = A.start[kk] + A.cnt[wave][kk] + rank;
     int* sorted = kk < S ? g.sorted_hot : g.sorted_cold;
@@ -217,44 +235,76 @@ __device__ __forceinline__ void align_rest(const AlignArgs& g, int mk, BlockDiv 
   fill_i32(g.eids_cold, min(d.div(t.cold), g.NB), g.NB, -1, me, n);
 }
 
-// One workgroup: T >= E, S and mk.
+// align_place for up to 64 ids, in one wave's registers: lane -> id `lane` of bucket `kk`. The
+// ids are sorted by (bucket, token); a bucket is then a run of lanes, and one scan over the
+// padded lengths of the runs gives every position.
+__device__ __forceinline__ AlignTotals align_place_wave(const AlignArgs& g, int S, BlockDiv d,
+                                                        int kk) {
+  const int lane = __lane_id();
+  const unsigned none = 0xFFFFFFFFu;
+  const unsigned s = wave_sort(kk >= 0 ? (unsigned)kk << 6 | (unsigned)lane : none);
+  const int b = (int)(s >> 6);
+  const bool valid = s != none;
+  const int prev = __builtin_amdgcn_update_dpp(-1, b, 0x138, 0xF, 0xF, false);  // lane - 1's
+  const unsigned long long heads = __ballot(valid & (b != prev));
+  const unsigned long long upto = lanes_below() << 1 | 1ull;  // this lane and those below
+  const int head = 63 - __clzll((long long)(heads & upto));
+  const unsigned long long later = heads & ~upto;
+  const int nvalid = (int)__popcll(__ballot(valid));
+  const int next = later ? __ffsll((long long)later) - 1 : nvalid;
+  const int padded = d.pad(next - head);
+  const bool first = valid & (b != prev);
+  const int scan = wave_incl_scan(first ? padded : 0);
+  const int nhot = (int)__popcll(__ballot(valid & (b < S)));
+  const int all = __builtin_amdgcn_readlane(scan, kWave - 1);
+  const int at = __builtin_amdgcn_readlane(scan, max(nhot - 1, 0));
+  const int hot = nhot > 0 ? at : 0;
+  if (valid) {
+    const bool is_hot = b < S;
+    const int start = scan - padded - (is_hot ? 0 : hot);
+    int* sorted = is_hot ? g.sorted_hot : g.sorted_cold;
+    const int pos = start + lane - head;
+    if (pos < g.L) sorted[pos] = (int)(s & 63);
+    if (first) {
+      int* eids = is_hot ? g.eids_hot : g.eids_cold;
+      const int q1 = min(d.div(start + padded), g.NB);
+      for (int q = d.div(start); q < q1; ++q) eids[q] = is_hot ? b : b - S;
+    }
+  }
+  return {hot, all - hot};
+}
+
+// One workgroup: T >= E, S and mk. All outputs get their defaults while the policy step's
+// loads are in flight (the step's second sync waits for those stores); the ids and the
+// blocks' experts are then stored over them, so padding needs no pass of its own.
 template <int W>
 __global__ __launch_bounds__(W* kWave) void fused_k(ManageArgs a, AlignArgs g) {
   constexpr int T = W * kWave;
   __shared__ ManageLds<W, false> L;
   __shared__ AlignLds<W> A;
-  // per side, the bucket of each block below the padded total: no more blocks than ids
-  __shared__ unsigned short block[2][T];
   args_in_sgprs(a);
   const int tid = threadIdx.x;
   const int E = a.E, S = a.S, mk = a.mk, waves = (mk + kWave - 1) / kWave;
-  const BlockDiv d(g.bs);
-  align_clear<W>(A, max(waves, 1), S + E);
+  const BlockDiv d(g);
   long long idv;
-  manage_step<W, false, 4>(a, L, idv);
+  manage_step<W, false, 4>(a, L, idv, [&] {
+    fill_i32(g.sorted_hot, 0, g.L, mk, tid, T);
+    fill_i32(g.sorted_cold, 0, g.L, mk, tid, T);
+    fill_i32(g.eids_hot, 0, g.NB, -1, tid, T);
+    fill_i32(g.eids_cold, 0, g.NB, -1, tid, T);
+    if (mk > kWave) align_clear<W>(A, waves, S + E);
+  });
   lds_sync();
-  const int kk = align_key((int)idv, E, S, L.tab);
-  const AlignTotals t = align_place<W, false>(g, A, E, S, d, kk, tid, max(waves, 1));
-  align_rest(g, mk, d, t, tid, T);
-  // thread b names the blocks of its two buckets
-  if (tid < S)
-    for (int q = d.div(A.start[tid]), q1 = d.div(A.end[tid] + g.bs - 1); q < q1; ++q)
-      block[0][q] = (unsigned short)tid;
-  if (tid < E)
-    for (int q = d.div(A.start[S + tid]), q1 = d.div(A.end[S + tid] + g.bs - 1); q < q1; ++q)
-      block[1][q] = (unsigned short)tid;
-  lds_sync();
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int total = h ? t.cold : t.hot;
-    const int* end = A.end + (h ? S : 0);
-    int* sorted = h ? g.sorted_cold : g.sorted_hot;
-    int* eids = h ? g.eids_cold : g.eids_hot;
-    const int q1 = min(d.div(total), g.NB);
-    for (int q = tid; q < q1; q += T) eids[q] = block[h][q];
-    const int p1 = min(total, g.L);
-    for (int p = tid; p < p1; p += T)
-      if (p >= end[block[h][d.div(p)]]) sorted[p] = mk;
+  AlignTotals t;
+  if (mk <= kWave) {
+    if (wave_index() != 0) return;
+    t = align_place_wave(g, S, d, align_key((int)idv, E, S, L.tab));
+  } else {
+    t = align_place<W, false>(g, A, E, S, d, align_key((int)idv, E, S, L.tab), tid, waves);
+  }
+  if (tid == 0) {
+    g.npad_hot[0] = t.hot;
+    g.npad_cold[0] = t.cold;
   }
 }
 
@@ -267,7 +317,7 @@ __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, i
   __shared__ unsigned short bucket[T];  // of each expert
   const int tid = threadIdx.x, part = blockIdx.x, parts = gridDim.x;
   const int first = part * T;
-  const BlockDiv d(g.bs);
+  const BlockDiv d(g);
   if (tid < E) {
     const int s = table[tid];
     bucket[tid] = (unsigned short)((unsigned)s < (unsigned)S ? s : S + tid);
@@ -276,28 +326,35 @@ __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, i
   A.start[tid] = A.start[T + tid] = A.end[tid] = A.end[T + tid] = 0;
   lds_sync();
   // ids of the other workgroups, counted per bucket: before this one's, and after
-  auto count = [&](int e, int i) {
-    if (e >= 0 && e < E) atomicAdd(&(i < first ? A.start : A.end)[bucket[e]], 1);
+  auto count = [&](int e, unsigned i) {
+    if (e >= 0 && e < E) atomicAdd(&(i < (unsigned)first ? A.start : A.end)[bucket[e]], 1);
   };
   const int mine = first + tid < mk ? ids[first + tid] : -1;
+  unsigned done = 0;  // ids counted
   if ((reinterpret_cast<uintptr_t>(ids) & 15) == 0) {
-    // four ids a load; `first` is a multiple of four and only the last workgroup's ids end
-    // at mk, so no vector straddles a boundary except the one cut off here
-    const int n4 = mk & ~3;
-    for (int i = 4 * tid; i < n4; i += 4 * T) {
-      if (i >= first && i < first + T) continue;
-      const i32x4 e = *reinterpret_cast<const i32x4*>(ids + i);
-      count(e.x, i);
-      count(e.y, i);
-      count(e.z, i);
-      count(e.w, i);
+    // four ids a load and four loads in flight; `first` is a multiple of four, and the
+    // workgroup's own ids end at a multiple of four or at mk
+    const i32x4* v = reinterpret_cast<const i32x4*>(ids);
+    const unsigned n = (unsigned)mk / 4;
+    for (unsigned i = tid; i < n; i += 4 * T) {
+      i32x4 e[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) e[k] = v[min(i + k * T, n - 1)];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const unsigned j = 4 * (i + k * T);
+        if (j < 4 * n && (j < (unsigned)first || j >= (unsigned)first + T)) {
+          count(e[k].x, j);
+          count(e[k].y, j);
+          count(e[k].z, j);
+          count(e[k].w, j);
+        }
+      }
     }
-    const int i = n4 + tid;
-    if (i < mk && (i < first || i >= first + T)) count(ids[i], i);
-  } else {
-    for (int i = tid; i < mk; i += T)
-      if (i < first || i >= first + T) count(ids[i], i);
+    done = 4 * n;
   }
+  for (unsigned i = done + tid; i < (unsigned)mk; i += T)
+    if (i < (unsigned)first || i >= (unsigned)first + T) count(ids[i], i);
   lds_sync();
   // positions of the buckets' starts: align_place leaves this workgroup's own in A.start
   int before[2] = {tid < S ? A.start[tid] : 0, tid < E ? A.start[S + tid] : 0};

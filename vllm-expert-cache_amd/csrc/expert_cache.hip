@@ -230,7 +230,7 @@ int expert_cache_fused(const int* topk_ids, int mk, int E, int S, int max_distin
                                  slot_expert, slot_stamp, routed, step, miss, n_miss, 0, 0,
                                  nullptr);
   AlignArgs g;
-  g.bs = bs;
+  set_block_size(g, bs);
   g.L = L;
   g.NB = NB;
   g.sorted_hot = sorted_hot;

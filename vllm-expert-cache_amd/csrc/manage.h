@@ -73,6 +73,8 @@ struct ManageLds {
   int wsum[2][W], wev[W];
 };
 
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
 template <int IDB>
 __device__ __forceinline__ long long load_id(const void* p, int i) {
   if constexpr (IDB == 8)
@@ -138,6 +140,11 @@ __device__ __forceinline__ long long uniform_i64(long long v) {
   return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
+// What a caller has the workgroup do between issuing the step's loads and needing them.
+struct NothingEarly {
+  __device__ __forceinline__ void operator()() const {}
+};
+
 // One policy step. On return, the updated table is in L.tab (or in memory for GLOBAL_E),
 // behind a sync that the caller makes, and idv holds ids[threadIdx.x] (or -1 past mk).
 //
@@ -152,9 +159,13 @@ __device__ __forceinline__ long long uniform_i64(long long v) {
 // whose expert is not routed is dropped -- the expert leaves the table and the slot is left
 // empty at stamp 0, so a prefetch copy still in flight may stop short. The reference never
 // holds a negative stamp, so on its states none of this runs.
-template <int W, bool GLOBAL_E, int IDB, bool PF = false>
+//
+// `early` runs once the loads are issued; its stores have completed, for every wave, before
+// the step's own, and before the step returns.
+template <int W, bool GLOBAL_E, int IDB, bool PF = false, class Early = NothingEarly>
 __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GLOBAL_E>& L,
-                                            long long& idv) {
+                                            long long& idv, const Early& early = Early()) {
+  static_assert(!GLOBAL_E || std::is_same<Early, NothingEarly>::value);
   static_assert(!PF || IDB == 4, "prefetch takes int32 ids");
   static_assert(!GLOBAL_E || W == 16, "insert lists of 1024 experts");
   constexpr int T = W * kWave;
@@ -184,6 +195,8 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   int tv = -1;
   if constexpr (!GLOBAL_E) tv = a.table[min(tid, E - 1)];
 
+  early();
+
   // clears: four bytes a thread
   unsigned char* flag;
   if constexpr (GLOBAL_E) {
@@ -205,13 +218,38 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const int e = (int)idv;
     if (e >= 0 && e < E) flag[e] = 1;
   }
-  for (unsigned i = tid + T; (int)i < mk; i += 4 * T) {
-    int e[4];
+  if (mk > T) {
+    const auto mark = [&](int e) {
+      if (e >= 0 && e < E) flag[e] = 1;
+    };
+    unsigned done = T;  // ids marked
+    if constexpr (IDB == 4) {
+      // four ids a load and four loads in flight; the first T ids are marked once more
+      if ((reinterpret_cast<uintptr_t>(a.ids) & 15) == 0) {
+        const i32x4* v = reinterpret_cast<const i32x4*>(a.ids);
+        const unsigned n = (unsigned)mk / 4;
+        for (unsigned i = tid; i < n; i += 4 * T) {
+          i32x4 e[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) e[k] = (int)ip[min(i + k * T, (unsigned)(mk - 1))];
+          for (int k = 0; k < 4; ++k) e[k] = v[min(i + k * T, n - 1)];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (e[k] >= 0 && e[k] < E) flag[e[k]] = 1;
+          for (int k = 0; k < 4; ++k) {
+            mark(e[k].x);
+            mark(e[k].y);
+            mark(e[k].z);
+            mark(e[k].w);
+          }
+        }
+        done = 4 * n;
+      }
+    }
+    for (unsigned i = done + tid; i < (unsigned)mk; i += 4 * T) {
+      int e[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) e[k] = (int)ip[min(i + k * T, (unsigned)(mk - 1))];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) mark(e[k]);
+    }
   }
   if constexpr (!GLOBAL_E) L.tab[tid] = tv;  // entries past E are written too: nothing reads them
   step_sync<GLOBAL_E>();
@@ -223,7 +261,6 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   int total = 0, distinct = 0;
   if constexpr (!GLOBAL_E) {
     const unsigned char fb = flag[tid];  // zero past E
-    if (tid < E) a.routed[tid] = fb;
     const bool m = (fb != 0) & (tv < 0);
     if (!PF && fb != 0 && tv >= 0 && tv < S) L.hit[tv] = 1;
     const unsigned long long mask = __ballot(m);
@@ -238,7 +275,15 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     if constexpr (W > 1) {
       if (lane == 0) L.wsum[0][wave] = mine;
     }
-    lds_sync();
+    // no store of the step's own precedes this sync: where `early` made some, they have had
+    // the load's round trip to complete, and waiting for them here costs little
+    if constexpr (std::is_same<Early, NothingEarly>::value) {
+      if (tid < E) a.routed[tid] = fb;
+      lds_sync();
+    } else {
+      mem_sync();
+      if (tid < E) a.routed[tid] = fb;
+    }
     if constexpr (W > 1) wave_sums<W>(L.wsum[0], wave, before, all);
     distinct = all >> 16;
     total = all & 0xFFFF;
@@ -344,7 +389,8 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const bool few = nins <= few_inserts<W>(S);
     int r = -1;  // insert this thread's slot takes
     if constexpr (W > 1) {
-      const unsigned sorted = few ? key : wave_sort(key);
+      // waves without slots have nothing to sort
+      const unsigned sorted = few || wave * kWave >= S ? key : wave_sort(key);
       L.key[tid] = sorted;
       L.ins[tid] = -1;
       if (lane == 0) L.wev[wave] = nev_wave;

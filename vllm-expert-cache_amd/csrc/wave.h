@@ -170,16 +170,19 @@ __device__ __forceinline__ unsigned wave_merge_low(unsigned v, unsigned down) {
 // bits (all lanes must be active). One ballot per bit: needs no LDS, and no order among the
 // lanes is assumed.
 __device__ __forceinline__ unsigned long long wave_match(int v, int bits) {
-  unsigned long long m = __ballot(v >= 0);
+  const unsigned long long valid = __ballot(v >= 0);
+  unsigned lo = (unsigned)valid, hi = (unsigned)(valid >> 32);
 #pragma unroll 1
-  for (int b = 0; b < bits; b += 4) {
+  for (int b = 0; b < bits; b += 3) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int bit = (v >> (b + k)) & 1;
-      m &= __ballot(bit) ^ ((unsigned long long)(long long)(bit - 1));
+    for (int k = 0; k < 3; ++k) {
+      const int bit = __builtin_amdgcn_sbfe(v, b + k, 1);  // 0 or -1
+      const unsigned long long set = __ballot(bit != 0);
+      lo &= ~((unsigned)set ^ (unsigned)bit);
+      hi &= ~((unsigned)(set >> 32) ^ (unsigned)bit);
     }
   }
-  return m;
+  return (unsigned long long)hi << 32 | lo;
 }
 
 // Sums over the waves of a workgroup, from one word per wave in LDS (W <= 16): the words of
