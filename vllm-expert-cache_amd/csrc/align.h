@@ -16,7 +16,8 @@
 //  * fused_k, up to kFusedIds ids: the policy step and both alignments in one workgroup,
 //    one id, one expert and one slot a thread. Up to 64 ids are placed by one wave that
 //    sorts them in registers.
-//  * align_k, more ids: a workgroup per 1024 ids, after a launch of the policy step alone.
+//  * align_k, more ids: a workgroup per 1024 ids, after a launch whose first workgroup runs
+//    the policy step while the others store the outputs' defaults (manage_defaults_k).
 //    Each workgroup counts the ids before and after its own itself (they come from the L2),
 //    which costs less than the node or the cross-XCD handoff that sharing the counts would.
 //
@@ -49,7 +50,7 @@ struct AlignLds {
   static constexpr int T = W * kWave;
   unsigned short cnt[W][2 * T];  // ids per bucket of each wave, then of the waves before it
   int start[2 * T];  // position of the workgroup's first id of the bucket
-  int end[2 * T];    // position past the bucket's last id
+  int end[2 * T];    // ids of the bucket after the workgroup's
   int wsum[2][W];
 };
 
@@ -87,20 +88,24 @@ struct BlockDiv {
   __device__ __forceinline__ int pad(int x) const { return div(x + bs - 1) * bs; }
 };
 
-// dst[from, to) = v over `n` threads of which this is number `me`; 16-byte stores when dst is
-// 16-byte aligned.
-__device__ __forceinline__ void fill_i32(int* dst, int from, int to, int v, int me, int n) {
-  if (from >= to) return;
-  if ((reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-    const int a0 = min((from + 3) & ~3, to);
-    const int a1 = a0 + ((to - a0) & ~3);
-    if (me < a0 - from) dst[from + me] = v;
-    for (long long p = a0 + 4ll * me; p < a1; p += 4ll * n)
-      *reinterpret_cast<i32x4*>(dst + p) = i32x4{v, v, v, v};
-    if (me < to - a1) dst[a1 + me] = v;
-  } else {
-    for (long long p = from + me; p < to; p += n) dst[p] = v;
+// x[0, n) = y[0, n) = v over `threads` threads of which this is number `me`; 16-byte stores
+// where both are 16-byte aligned.
+__device__ __forceinline__ void fill_pair(int* x, int* y, int n, int v, int me, int threads) {
+  unsigned p = 0;
+  if (((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0) {
+    const unsigned n4 = (unsigned)n / 4;
+    for (p = me; p < n4; p += threads) reinterpret_cast<i32x4*>(x)[p] = i32x4{v, v, v, v};
+    for (p = me; p < n4; p += threads) reinterpret_cast<i32x4*>(y)[p] = i32x4{v, v, v, v};
+    p = 4 * n4;
   }
+  for (p += me; p < (unsigned)n; p += threads) x[p] = y[p] = v;
+}
+
+// The defaults of all outputs: mk and -1.
+__device__ __forceinline__ void align_defaults(const AlignArgs& g, int mk, int me,
+                                               int threads) {
+  fill_pair(g.sorted_hot, g.sorted_cold, g.L, mk, me, threads);
+  fill_pair(g.eids_hot, g.eids_cold, g.NB, -1, me, threads);
 }
 
 // Clears the rows of the count matrix that `waves` waves fill; the caller syncs.
@@ -113,15 +118,14 @@ __device__ __forceinline__ void align_clear(AlignLds<W>& A, int waves, int bucke
 }
 
 // Places id `i` of bucket `kk` (-1: none) for every thread of the workgroup, whose ids are
-// consecutive and lie in its first `waves` waves. The count matrix is clear. With PART the
-// workgroup holds only some of the ids: on entry A.start and A.end hold, per bucket, the
-// counts of the ids before and after its own; on return A.end and, per bucket, A.start are
-// positions as declared (behind the sync made here). Without it, the blocks' expert ids are
-// written too.
+// consecutive and lie in its first `waves` waves, and names the blocks of the buckets. The
+// count matrix is clear and the outputs hold their defaults. With PART the workgroup is
+// number `part` of `parts` and holds only some of the ids: on entry A.start and A.end hold,
+// per bucket, the counts of the ids before and after its own.
 template <int W, bool PART>
 __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<W>& A, int E,
                                                    int S, BlockDiv d, int kk, int i,
-                                                   int waves) {
+                                                   int waves, int part, int parts) {
   const int tid = threadIdx.x, lane = __lane_id(), wave = wave_index();
   int rank = 0;
   if (wave < waves) {
@@ -181,17 +185,28 @@ __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<
     if (tid < size[h]) {
       const int b = tid + (h ? S : 0);
       A.start[b] = first[h] + before[h];
-      if constexpr (PART) A.end[b] = first[h] + n[h];
     }
   }
   lds_sync();
-  if constexpr (!PART) {
-    // thread b names the blocks of its two buckets
+  // Thread b names the blocks of its two buckets; the first workgroups of a launch, as many
+  // as a power of two, take each its share of every wave's buckets. A bucket of many blocks
+  // is left to its whole wave.
+  const int sharing = min(1 << (31 - __clz(parts)), kWave);
+  if (part < sharing) {
+    const bool own = (lane & (sharing - 1)) == part;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       int* eids = h ? g.eids_cold : g.eids_hot;
-      const int q1 = min(d.div(first[h] + padded[h]), g.NB);
-      for (int q = d.div(first[h]); q < q1; ++q) eids[q] = tid;
+      const int q0 = d.div(first[h]), q1 = min(d.div(first[h] + padded[h]), g.NB);
+      const bool many = own && q1 - q0 > 8;
+      if (own && !many)
+        for (int q = q0; q < q1; ++q) eids[q] = tid;
+      for (unsigned long long m = __ballot(many); m != 0; m &= m - 1) {
+        const int l = __ffsll((long long)m) - 1;
+        const int end = __builtin_amdgcn_readlane(q1, l);
+        for (int q = __builtin_amdgcn_readlane(q0, l) + lane; q < end; q += kWave)
+          eids[q] = wave * kWave + l;
+      }
     }
   }
   if (kk >= 0) {
@@ -202,47 +217,15 @@ __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<
   return {total[0], total[1]};
 }
 
-// The padding of each bucket (mk) and its blocks' expert ids, a wave per bucket of the
-// launch's `nwaves`, this one being number `me`. `from` is the bucket's first position.
-template <int W>
-__device__ __forceinline__ void align_pad(const AlignArgs& g, const AlignLds<W>& A, int E,
-                                          int S, int mk, BlockDiv d, int me, int nwaves,
-                                          const int* from) {
-  const int lane = __lane_id();
-  for (int b = me; b < S + E; b += nwaves) {
-    const int p0 = from[b], p1 = A.end[b];
-    if (p0 == p1) continue;
-    const int p2 = p0 + d.pad(p1 - p0);
-    int* sorted = b < S ? g.sorted_hot : g.sorted_cold;
-    int* eids = b < S ? g.eids_hot : g.eids_cold;
-    const int id = b < S ? b : b - S;
-    for (int p = p1 + lane; p < min(p2, g.L); p += kWave) sorted[p] = mk;
-    const int q1 = min(d.div(p2), g.NB);
-    for (int q = d.div(p0) + lane; q < q1; q += kWave) eids[q] = id;
-  }
-}
-
-// Past the padded totals the outputs hold mk and -1.
-__device__ __forceinline__ void align_rest(const AlignArgs& g, int mk, BlockDiv d,
-                                           AlignTotals t, int me, int n) {
-  if (me == 0) {
-    g.npad_hot[0] = t.hot;
-    g.npad_cold[0] = t.cold;
-  }
-  fill_i32(g.sorted_hot, min(t.hot, g.L), g.L, mk, me, n);
-  fill_i32(g.sorted_cold, min(t.cold, g.L), g.L, mk, me, n);
-  fill_i32(g.eids_hot, min(d.div(t.hot), g.NB), g.NB, -1, me, n);
-  fill_i32(g.eids_cold, min(d.div(t.cold), g.NB), g.NB, -1, me, n);
-}
-
 // align_place for up to 64 ids, in one wave's registers: lane -> id `lane` of bucket `kk`. The
 // ids are sorted by (bucket, token); a bucket is then a run of lanes, and one scan over the
 // padded lengths of the runs gives every position.
-__device__ __forceinline__ AlignTotals align_place_wave(const AlignArgs& g, int S, BlockDiv d,
-                                                        int kk) {
+__device__ __forceinline__ AlignTotals align_place_wave(const AlignArgs& g, int S, int mk,
+                                                        BlockDiv d, int kk) {
   const int lane = __lane_id();
   const unsigned none = 0xFFFFFFFFu;
-  const unsigned s = wave_sort(kk >= 0 ? (unsigned)kk << 6 | (unsigned)lane : none);
+  const unsigned key = kk >= 0 ? (unsigned)kk << 6 | (unsigned)lane : none;
+  const unsigned s = mk <= 16 ? row_sort(key) : wave_sort(key);
   const int b = (int)(s >> 6);
   const bool valid = s != none;
   const int prev = __builtin_amdgcn_update_dpp(-1, b, 0x138, 0xF, 0xF, false);  // lane - 1's
@@ -288,19 +271,17 @@ __global__ __launch_bounds__(W* kWave) void fused_k(ManageArgs a, AlignArgs g) {
   const BlockDiv d(g);
   long long idv;
   manage_step<W, false, 4>(a, L, idv, [&] {
-    fill_i32(g.sorted_hot, 0, g.L, mk, tid, T);
-    fill_i32(g.sorted_cold, 0, g.L, mk, tid, T);
-    fill_i32(g.eids_hot, 0, g.NB, -1, tid, T);
-    fill_i32(g.eids_cold, 0, g.NB, -1, tid, T);
+    align_defaults(g, mk, tid, T);
     if (mk > kWave) align_clear<W>(A, waves, S + E);
   });
   lds_sync();
   AlignTotals t;
   if (mk <= kWave) {
     if (wave_index() != 0) return;
-    t = align_place_wave(g, S, d, align_key((int)idv, E, S, L.tab));
+    t = align_place_wave(g, S, mk, d, align_key((int)idv, E, S, L.tab));
   } else {
-    t = align_place<W, false>(g, A, E, S, d, align_key((int)idv, E, S, L.tab), tid, waves);
+    t = align_place<W, false>(g, A, E, S, d, align_key((int)idv, E, S, L.tab), tid, waves, 0,
+                              1);
   }
   if (tid == 0) {
     g.npad_hot[0] = t.hot;
@@ -308,12 +289,12 @@ __global__ __launch_bounds__(W* kWave) void fused_k(ManageArgs a, AlignArgs g) {
   }
 }
 
-// A workgroup per 1024 ids, against the table as it is.
+// A workgroup per 1024 ids, against the table as it is, over outputs that hold their
+// defaults.
 __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, int S,
                                                 const int* table, AlignArgs g) {
   constexpr int W = 16, T = W * kWave;
   __shared__ AlignLds<W> A;
-  __shared__ int from[2 * T];           // first position of each bucket
   __shared__ unsigned short bucket[T];  // of each expert
   const int tid = threadIdx.x, part = blockIdx.x, parts = gridDim.x;
   const int first = part * T;
@@ -356,15 +337,26 @@ __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, i
   for (unsigned i = done + tid; i < (unsigned)mk; i += T)
     if (i < (unsigned)first || i >= (unsigned)first + T) count(ids[i], i);
   lds_sync();
-  // positions of the buckets' starts: align_place leaves this workgroup's own in A.start
-  int before[2] = {tid < S ? A.start[tid] : 0, tid < E ? A.start[S + tid] : 0};
   const int kk = mine >= 0 && mine < E ? bucket[mine] : -1;
-  const AlignTotals t = align_place<W, true>(g, A, E, S, d, kk, first + tid, W);
-  if (tid < S) from[tid] = A.start[tid] - before[0];
-  if (tid < E) from[S + tid] = A.start[S + tid] - before[1];
-  lds_sync();
-  align_rest(g, mk, d, t, first + tid, parts * T);
-  align_pad<W>(g, A, E, S, mk, d, part * W + wave_index(), parts * W, from);
+  const AlignTotals t = align_place<W, true>(g, A, E, S, d, kk, first + tid, W, part, parts);
+  if (part == 0 && tid == 0) {
+    g.npad_hot[0] = t.hot;
+    g.npad_cold[0] = t.cold;
+  }
+}
+
+// The policy step in the launch's first workgroup; the others store the alignments' defaults.
+template <int W>
+__global__ __launch_bounds__(W* kWave) void manage_defaults_k(ManageArgs a, AlignArgs g) {
+  __shared__ ManageLds<W, false> L;
+  if (blockIdx.x > 0) {
+    align_defaults(g, a.mk, (blockIdx.x - 1) * W * kWave + threadIdx.x,
+                   (gridDim.x - 1) * W * kWave);
+    return;
+  }
+  args_in_sgprs(a);
+  long long idv;
+  manage_step<W, false, 4>(a, L, idv);
 }
 
 }  // namespace ec

@@ -100,7 +100,13 @@ int launch_fused(const ManageArgs& a, const AlignArgs& g, hipStream_t stream) {
     });
     return (int)hipGetLastError();
   }
-  const int rc = launch_manage<4, false>(a, stream);
+  // the fills get a workgroup per 16 K outputs a side
+  const int fills = g.L / 16384 < 255 ? g.L / 16384 + 1 : 256;
+  with_waves(waves_for(a.E, a.S, a.mk), [&](auto w) {
+    hipLaunchKernelGGL((manage_defaults_k<w()>), dim3(1 + fills), dim3(w() * kWave), 0, stream,
+                       a, g);
+  });
+  const int rc = (int)hipGetLastError();
   if (rc) return rc;
   hipLaunchKernelGGL(align_k, dim3((a.mk - 1) / 1024 + 1), dim3(1024), 0, stream,
                      static_cast<const int*>(a.ids), a.mk, a.E, a.S, a.table, g);

@@ -126,9 +126,9 @@ __device__ __forceinline__ unsigned sort_step(unsigned v) {
   return (__lane_id() & B) ? max(v, o) : min(v, o);
 }
 
-// `v` sorted ascending over the 64 lanes: 21 compare-exchanges in registers. Each merge
-// starts with a mirrored exchange, so all of them run in ascending order.
-__device__ __forceinline__ unsigned wave_sort(unsigned v) {
+// `v` sorted ascending over each row of 16 lanes: 10 compare-exchanges in registers. Each
+// merge starts with a mirrored exchange, so all of them run in ascending order.
+__device__ __forceinline__ unsigned row_sort(unsigned v) {
   v = sort_step<1, 1>(v);
   v = sort_step<3, 2>(v);
   v = sort_step<1, 1>(v);
@@ -139,6 +139,12 @@ __device__ __forceinline__ unsigned wave_sort(unsigned v) {
   v = sort_step<4, 4>(v);
   v = sort_step<2, 2>(v);
   v = sort_step<1, 1>(v);
+  return v;
+}
+
+// `v` sorted ascending over the 64 lanes: 11 more.
+__device__ __forceinline__ unsigned wave_sort(unsigned v) {
+  v = row_sort(v);
   v = sort_step<31, 16>(v);
   v = sort_step<8, 8>(v);
   v = sort_step<4, 4>(v);
