@@ -295,22 +295,28 @@ __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, i
                                                 const int* table, AlignArgs g) {
   constexpr int W = 16, T = W * kWave;
   __shared__ AlignLds<W> A;
-  __shared__ unsigned short bucket[T];  // of each expert
+  __shared__ unsigned short expert_bucket[T];
+  // ids of the other workgroups per expert, before this one's ids and after: four counts of
+  // each, by lane, so that a popular expert's ids do not all meet at one address
+  __shared__ i32x4 count[2][T];
   const int tid = threadIdx.x, part = blockIdx.x, parts = gridDim.x;
-  const int first = part * T;
+  const unsigned first = part * T;
   const BlockDiv d(g);
+  int bucket = -1;  // of expert `tid`
   if (tid < E) {
     const int s = table[tid];
-    bucket[tid] = (unsigned short)((unsigned)s < (unsigned)S ? s : S + tid);
+    bucket = (unsigned)s < (unsigned)S ? s : S + tid;
   }
+  const int mine = first + tid < (unsigned)mk ? ids[first + tid] : -1;
   align_clear<W>(A, W, S + E);
   A.start[tid] = A.start[T + tid] = A.end[tid] = A.end[T + tid] = 0;
+  count[0][tid] = count[1][tid] = i32x4{0, 0, 0, 0};
   lds_sync();
-  // ids of the other workgroups, counted per bucket: before this one's, and after
-  auto count = [&](int e, unsigned i) {
-    if (e >= 0 && e < E) atomicAdd(&(i < (unsigned)first ? A.start : A.end)[bucket[e]], 1);
+  const int copy = tid & 3;
+  auto add = [&](int e, unsigned i) {
+    if ((unsigned)e < (unsigned)E)
+      atomicAdd(reinterpret_cast<int*>(&count[i < first ? 0 : 1][e]) + copy, 1);
   };
-  const int mine = first + tid < mk ? ids[first + tid] : -1;
   unsigned done = 0;  // ids counted
   if ((reinterpret_cast<uintptr_t>(ids) & 15) == 0) {
     // four ids a load and four loads in flight; `first` is a multiple of four, and the
@@ -324,20 +330,27 @@ __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, i
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const unsigned j = 4 * (i + k * T);
-        if (j < 4 * n && (j < (unsigned)first || j >= (unsigned)first + T)) {
-          count(e[k].x, j);
-          count(e[k].y, j);
-          count(e[k].z, j);
-          count(e[k].w, j);
+        if (j < 4 * n && (j < first || j >= first + T)) {
+          add(e[k].x, j);
+          add(e[k].y, j);
+          add(e[k].z, j);
+          add(e[k].w, j);
         }
       }
     }
     done = 4 * n;
   }
   for (unsigned i = done + tid; i < (unsigned)mk; i += T)
-    if (i < (unsigned)first || i >= (unsigned)first + T) count(ids[i], i);
+    if (i < first || i >= first + T) add(ids[i], i);
   lds_sync();
-  const int kk = mine >= 0 && mine < E ? bucket[mine] : -1;
+  if (bucket >= 0) {
+    const i32x4 b = count[0][tid], c = count[1][tid];
+    atomicAdd(&A.start[bucket], b.x + b.y + b.z + b.w);
+    atomicAdd(&A.end[bucket], c.x + c.y + c.z + c.w);
+    expert_bucket[tid] = (unsigned short)bucket;
+  }
+  lds_sync();
+  const int kk = (unsigned)mine < (unsigned)E ? expert_bucket[mine] : -1;
   const AlignTotals t = align_place<W, true>(g, A, E, S, d, kk, first + tid, W, part, parts);
   if (part == 0 && tid == 0) {
     g.npad_hot[0] = t.hot;

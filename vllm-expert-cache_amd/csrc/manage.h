@@ -62,7 +62,8 @@ struct ManageArgs {
 template <int W, bool GLOBAL_E>
 struct ManageLds {
   static constexpr int T = W * kWave;
-  alignas(16) unsigned char flag[GLOBAL_E ? 16 : T];  // expert routed this step
+  // expert routed this step: a word each, so that the marks of many ids spread over the banks
+  int flag[GLOBAL_E ? 1 : T];
   alignas(16) unsigned char hit[T];  // slot refreshed by a routed expert this step
   int tab[GLOBAL_E ? 1 : T];
   unsigned key[T];      // victim keys (sorted within each wave where every wave sorts)
@@ -198,13 +199,13 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   early();
 
   // clears: four bytes a thread
-  unsigned char* flag;
+  typename std::conditional<GLOBAL_E, unsigned char, int>::type* flag;
   if constexpr (GLOBAL_E) {
     flag = a.routed;
     for (int e = tid; e < E; e += T) flag[e] = 0;
   } else {
     flag = L.flag;
-    if (tid < T / 4) reinterpret_cast<unsigned*>(L.flag)[tid] = 0;
+    flag[tid] = 0;
   }
   if (tid < T / 4) reinterpret_cast<unsigned*>(L.hit)[tid] = 0;
   step_sync<GLOBAL_E>();
@@ -260,7 +261,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   const bool fx = held & (flag[held ? se : 0] != 0);  // the slot's expert is routed
   int total = 0, distinct = 0;
   if constexpr (!GLOBAL_E) {
-    const unsigned char fb = flag[tid];  // zero past E
+    const int fb = flag[tid];  // zero past E
     const bool m = (fb != 0) & (tv < 0);
     if (!PF && fb != 0 && tv >= 0 && tv < S) L.hit[tv] = 1;
     const unsigned long long mask = __ballot(m);
@@ -278,11 +279,11 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     // no store of the step's own precedes this sync: where `early` made some, they have had
     // the load's round trip to complete, and waiting for them here costs little
     if constexpr (std::is_same<Early, NothingEarly>::value) {
-      if (tid < E) a.routed[tid] = fb;
+      if (tid < E) a.routed[tid] = (unsigned char)fb;
       lds_sync();
     } else {
       mem_sync();
-      if (tid < E) a.routed[tid] = fb;
+      if (tid < E) a.routed[tid] = (unsigned char)fb;
     }
     if constexpr (W > 1) wave_sums<W>(L.wsum[0], wave, before, all);
     distinct = all >> 16;
