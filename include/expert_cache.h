@@ -181,6 +181,39 @@ int expert_cache_manage_remap_prefetch(
     int* pf_slot_expert, long long* pf_slot_stamp, unsigned char* pf_routed, int* pf_miss,
     int* pf_n_miss, hipStream_t stream);
 
+/*
+ * One layer as expert_cache_refresh takes it: the shape, the policy, the state arrays above
+ * (miss of 2*S ints), and the gather's arguments. `arrived` is one unsigned of the layer's
+ * own on the device, zero before the first call; every call leaves it zero.
+ */
+typedef struct expert_cache_layer {
+  int E, S, policy, decay, chunks, lanes;
+  int* table;
+  int* map_cold;
+  int* slot_expert;
+  long long* slot_stamp;
+  unsigned char* routed;
+  long long* step;
+  int* miss;
+  int* n_miss;
+  unsigned* arrived;
+  void* dst[6];
+  const void* src[6];
+  long bytes[6];
+} expert_cache_layer;
+
+/*
+ * A decode step of one layer: expert_cache_manage_remap with max_distinct = min(E, mk) and
+ * max_inserts = S, followed by expert_cache_gather of its miss list, in one launch where
+ * E and S are at most 256 (two otherwise), with the same results as the two calls. `layer`
+ * is read during the call only; `out` must not overlap `ids`. Argument checks are those of the two calls, plus mk >= 0 and
+ * `arrived` non-null; nothing runs if one of them fails.
+ *
+ * Replaces: vllm_expert_cache/cache.py:112-163; no counterpart in the reference's C-ABI.
+ */
+int expert_cache_refresh(const expert_cache_layer* layer, const void* ids, int id_bytes, int mk,
+                         void* out, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -254,3 +254,26 @@ def test_manage_remap_prefetch_rejects(lib, over):
     """expert_cache_manage_remap_prefetch checks its arguments, and that the two layers'
     arrays are disjoint, on the host before any HIP call."""
     assert _manage_prefetch(lib, **over) == -1
+
+
+def test_refresh_refuses_what_its_two_calls_refuse(lib):
+    """expert_cache_refresh returns -1 before any HIP call for each bad field or argument."""
+    def layer(**bad):
+        f = {n: 1 for n, _ in _lib.Layer._fields_}
+        f.update(E=8, S=4, policy=1, decay=64, chunks=32, lanes=1, bytes=16)
+        f.update(bad)
+        for n, t in (("dst", P), ("src", P), ("bytes", ctypes.c_long)):
+            f[n] = (t * 6)(*[f[n]] * 6)
+        return _lib.Layer(**f)
+
+    def call(l, id_bytes=4, mk=1, out=1):
+        return lib.expert_cache_refresh(ctypes.addressof(l) if l else None, 1, id_bytes, mk,
+                                        out, None)
+
+    assert call(None) == -1
+    for bad in ({"E": 0}, {"S": 0}, {"S": 1025}, {"policy": 2}, {"policy": -1}, {"chunks": 0},
+                {"lanes": 0}, {"n_miss": None}, {"arrived": None}, {"bytes": 0}, {"bytes": 24}):
+        assert call(layer(**bad)) == -1, bad
+    assert call(layer(), id_bytes=2) == -1
+    assert call(layer(), mk=-1) == -1
+    assert call(layer(), out=None) == -1

@@ -107,3 +107,81 @@ def test_fused_at_the_workgroups_edges(mk, E, S, bs):
         for k, v in want.items():
             assert np.array_equal(outs[k].cpu().numpy(), v), (t, k)
         _check_state(st, ref, f"mk={mk} step {t}")
+
+
+@pytest.mark.parametrize("E,S", [(8, 4), (64, 64), (200, 130), (256, 256), (257, 100)])
+@pytest.mark.parametrize("chunks", [1, 7, 32, 300])
+@pytest.mark.parametrize("id64", [False, True])
+def test_refresh_matches_policy_step_and_gather(E, S, chunks, id64, monkeypatch):
+    """One-launch refreshes (one workgroup, fewer than the tiles, more than the CUs) beside the
+    separate calls on a twin, over steps with no, some and all slots replaced, read-through
+    steps and pending prefetches to settle; state, slot ids and slot bytes after every step."""
+    from types import SimpleNamespace
+
+    from vllm_expert_cache.cache import ExpertSlotCache
+
+    monkeypatch.setenv("EXPERT_CACHE_CHUNKS", str(chunks))
+    rng = np.random.default_rng(E + S + chunks)
+    sizes = [4096 * 3 + 16, 48, 8192 * 2, 16, 64, 32, 80]  # seven: a second gather call
+    owner = SimpleNamespace(**{f"w{i}": gu.pinned(E * n).view(E, n)
+                               for i, n in enumerate(sizes)})
+    for t in vars(owner).values():
+        gu.fill_random(t.view(-1), int(rng.integers(1 << 30)))
+    one, two = (ExpertSlotCache(owner, list(vars(owner)), E, S, gu.DEV) for _ in range(2))
+    for c in (one, two):
+        c.policy, c.decay = 1, 3
+        for t in c.slots.values():
+            t.zero_()
+    two._layer_plan = lambda: (None, None)  # the separate calls
+    dt = torch.int64 if id64 else torch.int32
+    for t in range(12):
+        k = int(rng.choice([1, 2, max(1, S // 2), S, E]))
+        ids = rng.permutation(E)[:k]
+        ids = torch.as_tensor(np.resize(ids, max(k, 3)), device=gu.DEV).to(dt)
+        ids[rng.integers(0, ids.numel())] = -1
+        if t % 4 == 3:
+            for c in (one, two):
+                c.prefetch(ids[:min(S, ids.numel())].roll(1) + 1)
+                c.join()
+        if t == 6:
+            for c in (one, two):
+                c.policy = 0
+        outs = [c.refresh(ids) for c in (one, two)]
+        torch.cuda.synchronize()
+        assert torch.equal(*outs), t
+        assert int(one.arrived) == 0
+        for f in ("table", "map_cold", "slot_expert", "slot_stamp", "routed", "step", "miss",
+                  "n_miss"):
+            assert torch.equal(getattr(one, f), getattr(two, f)), (t, f)
+        for n in one.names:
+            assert torch.equal(one.slots[n], two.slots[n]), (t, n)
+
+
+def test_refresh_in_a_graph():
+    """Captured refreshes of two layers, replayed with the eager twin's steps between."""
+    from types import SimpleNamespace
+
+    from vllm_expert_cache.cache import ExpertSlotCache
+
+    E, S, k = 96, 40, 12
+    rng = np.random.default_rng(9)
+    owner = SimpleNamespace(w=gu.pinned(E * 4112).view(E, 4112))
+    gu.fill_random(owner.w.view(-1), 1)
+    caches = [ExpertSlotCache(owner, ["w"], E, S, gu.DEV) for _ in range(4)]
+    for c in caches:
+        c.slots["w"].zero_()
+    ids = torch.zeros(2, k, dtype=torch.int32, device=gu.DEV)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        outs = [c.refresh(i) for c, i in zip(caches[:2], ids)]
+    for t in range(10):
+        ids.copy_(torch.as_tensor(np.stack([rng.permutation(E)[:k] for _ in range(2)])))
+        graph.replay()
+        want = [c.refresh(i) for c, i in zip(caches[2:], ids)]
+        torch.cuda.synchronize()
+        for l in range(2):
+            assert torch.equal(outs[l], want[l]), (t, l)
+            for f in ("table", "slot_expert", "slot_stamp", "step", "n_miss"):
+                assert torch.equal(getattr(caches[l], f), getattr(caches[l + 2], f)), (t, l, f)
+            assert torch.equal(caches[l].slots["w"], caches[l + 2].slots["w"]), (t, l)

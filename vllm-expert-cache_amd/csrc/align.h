@@ -270,10 +270,11 @@ __global__ __launch_bounds__(W* kWave) void fused_k(ManageArgs a, AlignArgs g) {
   const int E = a.E, S = a.S, mk = a.mk, waves = (mk + kWave - 1) / kWave;
   const BlockDiv d(g);
   long long idv;
-  manage_step<W, false, 4>(a, L, idv, [&] {
+  const auto early = [&] {
     align_defaults(g, mk, tid, T);
     if (mk > kWave) align_clear<W>(A, waves, S + E);
-  });
+  };
+  manage_step<W, false, 4>(a, L, idv, EarlyStep<decltype(early)>(early));
   lds_sync();
   AlignTotals t;
   if (mk <= kWave) {

@@ -13,6 +13,7 @@
 #include "align.h"
 #include "gather.h"
 #include "manage.h"
+#include "refresh.h"
 
 namespace ec {
 namespace {
@@ -246,6 +247,34 @@ int expert_cache_fused(const int* topk_ids, int mk, int E, int S, int max_distin
   g.eids_cold = eids_cold;
   g.npad_cold = npad_cold;
   return launch_fused(a, g, stream);
+}
+
+int expert_cache_refresh(const expert_cache_layer* c, const void* ids, int id_bytes, int mk,
+                         void* out, hipStream_t stream) {
+  if (c == nullptr || c->arrived == nullptr || mk < 0) return -1;
+  if (manage_args_bad(c->E, c->S, c->S, c->policy)) return -1;
+  if (id_bytes != 4 && id_bytes != 8) return -1;
+  if (mk > 0 && out == nullptr) return -1;
+  GatherArgs g;
+  if (c->n_miss == nullptr || !gather_plan(c->dst, c->src, c->bytes, c->chunks, c->lanes, g))
+    return -1;
+  const ManageArgs a = make_args(ids, mk, c->E, c->S, c->E < mk ? c->E : mk, c->S, c->table,
+                                 c->map_cold, c->slot_expert, c->slot_stamp, c->routed, c->step,
+                                 c->miss, c->n_miss, c->policy, c->decay, out);
+  const dim3 grid(c->chunks, c->lanes), block(kGatherThreads);
+  if (c->E <= kGatherThreads && c->S <= kGatherThreads) {
+    if (id_bytes == 8)
+      hipLaunchKernelGGL((refresh_k<8>), grid, block, 0, stream, a, g, c->arrived);
+    else
+      hipLaunchKernelGGL((refresh_k<4>), grid, block, 0, stream, a, g, c->arrived);
+    return (int)hipGetLastError();
+  }
+  const int rc = id_bytes == 8 ? launch_manage<8, true>(a, stream)
+                               : launch_manage<4, true>(a, stream);
+  if (rc) return rc;
+  hipLaunchKernelGGL((gather_k<kGatherUnroll, true, false, false>), grid, block, 0, stream, g,
+                     c->miss, c->n_miss, nullptr);
+  return (int)hipGetLastError();
 }
 
 int expert_cache_gather(void* d0, const void* s0, long b0, void* d1, const void* s1, long b1,

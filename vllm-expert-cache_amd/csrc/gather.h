@@ -104,20 +104,19 @@ __device__ __forceinline__ void tile_store(const GatherTile& t, const u32x4 (&v)
 // issued one tile ahead, so no tile load waits for it; the first tile of a miss is loaded
 // without one. Tiles already loaded are still stored: a dropped slot is empty, or gets
 // another expert whose own copy the caller orders after this kernel.
-template <int U, bool NT_LOAD, bool NT_STORE, bool LIVE>
-__device__ __forceinline__ void gather_walk(const GatherArgs& g, const int* __restrict__ miss,
-                                            const int* __restrict__ n_miss,
-                                            const int* slot_expert, long long t0) {
+//
+// `pair(j, e, sl)` gives the j-th pair of the list, j < nm.
+template <int U, bool NT_LOAD, bool NT_STORE, bool LIVE, class Pair>
+__device__ __forceinline__ void gather_pairs(const GatherArgs& g, int nm, const Pair& pair,
+                                             const int* slot_expert, long long t0) {
   const long long per = g.per;
-  // The miss list is read only below n_miss, as kernels/expert_cache.hip:294-298 reads it:
-  // a caller with no insert capacity (max_inserts = 0) may pass an empty list.
-  const int nm = n_miss[0];
   if (nm <= 0 || per <= 0 || t0 >= (long long)nm * per) return;
   const long long jstep = g.jstep, rstep = g.rstep;
   // first tile: in miss 0 whenever a miss spans more tiles than the grid has workgroups
   int j = t0 < per ? 0 : (int)(t0 / per);
   long long r = t0 - (long long)j * per;
-  int e = miss[2 * j], sl = miss[2 * j + 1];
+  int e, sl;
+  pair(j, e, sl);
   // slot_expert[sl] as last read, for the next tile of the same miss; every such read is
   // issued before the tile loads that follow it, so waiting for it never waits for them
   int seen = 0;
@@ -138,8 +137,7 @@ __device__ __forceinline__ void gather_walk(const GatherArgs& g, const int* __re
     if (jn >= nm) break;
     bool live = true;
     if (jn != j) {
-      e = miss[2 * jn];
-      sl = miss[2 * jn + 1];
+      pair(jn, e, sl);
       if constexpr (LIVE)
         seen = __hip_atomic_load(slot_expert + sl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else if constexpr (LIVE) {
@@ -164,6 +162,22 @@ __device__ __forceinline__ void gather_walk(const GatherArgs& g, const int* __re
     }
   }
   if (have) tile_store<U, NT_STORE>(cur, v);
+}
+
+// The walk over a miss list in memory. It is read only below n_miss, as
+// kernels/expert_cache.hip:294-298 reads it: a caller with no insert capacity
+// (max_inserts = 0) may pass an empty list.
+template <int U, bool NT_LOAD, bool NT_STORE, bool LIVE>
+__device__ __forceinline__ void gather_walk(const GatherArgs& g, const int* __restrict__ miss,
+                                            const int* __restrict__ n_miss,
+                                            const int* slot_expert, long long t0) {
+  gather_pairs<U, NT_LOAD, NT_STORE, LIVE>(
+      g, n_miss[0],
+      [&](int j, int& e, int& sl) {
+        e = miss[2 * j];
+        sl = miss[2 * j + 1];
+      },
+      slot_expert, t0);
 }
 
 template <int U, bool NT_LOAD, bool NT_STORE, bool LIVE>

@@ -69,6 +69,7 @@ struct ManageLds {
   unsigned key[T];      // victim keys (sorted within each wave where every wave sorts)
   int ins[T];           // slot -> insert it takes, or -1
   int mis[T];           // insert r -> missing expert
+  int vic[T];           // insert r -> slot, where the caller asks for it
   long long key64[T];   // 64-bit victim keys, where the stamps need them
   long long wmin[W];
   int wsum[2][W], wev[W];
@@ -141,9 +142,45 @@ __device__ __forceinline__ long long uniform_i64(long long v) {
   return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
-// What a caller has the workgroup do between issuing the step's loads and needing them.
-struct NothingEarly {
-  __device__ __forceinline__ void operator()() const {}
+// What one thread (expert `tid`, slot `tid`) has to store for a step. A kernel whose
+// workgroups all run the step has one of them store it, once all have read the state.
+struct StepStores {
+  bool served;      // past the read-through check
+  bool inserting;   // there were misses to insert, whether or not slots for them
+  int routed;       // the expert's flag
+  int miss;         // the expert's index in the miss list, or -1
+  int dropped;      // expert of a pending prefetch install that leaves the slot, or -1
+  int evicted;      // expert that leaves the slot for `expert`, or -1
+  int insert;       // insert the slot takes, or -1
+  int expert;       // ... and its expert
+  bool moved, aged; // slot_expert, slot_stamp change, to
+  int slot_expert;
+  long long slot_stamp, step;
+  int nact;
+};
+
+// What a caller adds to the step:
+//  kEarly  early() runs once the loads are issued; its stores have completed, for every
+//          wave, before the step's own, and before the step returns;
+//  kDefer  the step's global stores go into `stores` (and the inserts' slots to L.vic)
+//          instead of to memory, and every wave's loads have returned before the step does.
+struct PlainStep {
+  static constexpr bool kEarly = false, kDefer = false;
+  __device__ __forceinline__ void early() const {}
+};
+
+template <class F>
+struct EarlyStep : PlainStep {
+  static constexpr bool kEarly = true;
+  F f;
+  __device__ __forceinline__ explicit EarlyStep(const F& fn) : f(fn) {}
+  __device__ __forceinline__ void early() const { f(); }
+};
+
+struct DeferredStep : PlainStep {
+  static constexpr bool kDefer = true;
+  StepStores& stores;
+  __device__ __forceinline__ explicit DeferredStep(StepStores& s) : stores(s) {}
 };
 
 // One policy step. On return, the updated table is in L.tab (or in memory for GLOBAL_E),
@@ -160,13 +197,12 @@ struct NothingEarly {
 // whose expert is not routed is dropped -- the expert leaves the table and the slot is left
 // empty at stamp 0, so a prefetch copy still in flight may stop short. The reference never
 // holds a negative stamp, so on its states none of this runs.
-//
-// `early` runs once the loads are issued; its stores have completed, for every wave, before
-// the step's own, and before the step returns.
-template <int W, bool GLOBAL_E, int IDB, bool PF = false, class Early = NothingEarly>
+template <int W, bool GLOBAL_E, int IDB, bool PF = false, class Caller = PlainStep>
 __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GLOBAL_E>& L,
-                                            long long& idv, const Early& early = Early()) {
-  static_assert(!GLOBAL_E || std::is_same<Early, NothingEarly>::value);
+                                            long long& idv, const Caller& caller = Caller()) {
+  constexpr bool kDefer = Caller::kDefer;
+  static_assert(!GLOBAL_E || !(Caller::kEarly || kDefer));
+  static_assert(!PF || !kDefer);
   static_assert(!PF || IDB == 4, "prefetch takes int32 ids");
   static_assert(!GLOBAL_E || W == 16, "insert lists of 1024 experts");
   constexpr int T = W * kWave;
@@ -196,7 +232,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   int tv = -1;
   if constexpr (!GLOBAL_E) tv = a.table[min(tid, E - 1)];
 
-  early();
+  caller.early();
 
   // clears: four bytes a thread
   typename std::conditional<GLOBAL_E, unsigned char, int>::type* flag;
@@ -253,7 +289,9 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     }
   }
   if constexpr (!GLOBAL_E) L.tab[tid] = tv;  // entries past E are written too: nothing reads them
+  if constexpr (kDefer) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   step_sync<GLOBAL_E>();
+  StepStores keep{false, false, 0, -1, -1, -1, -1, 0, false, false, 0, 0, 0, 0};
 
   // ---- distinct count (the caller's `routed` is left holding the flags); hits mark their
   // ---- slot; misses enumerate in ascending expert id ----------------------------------
@@ -278,20 +316,22 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     }
     // no store of the step's own precedes this sync: where `early` made some, they have had
     // the load's round trip to complete, and waiting for them here costs little
-    if constexpr (std::is_same<Early, NothingEarly>::value) {
-      if (tid < E) a.routed[tid] = (unsigned char)fb;
-      lds_sync();
-    } else {
-      mem_sync();
-      if (tid < E) a.routed[tid] = (unsigned char)fb;
-    }
+    if constexpr (Caller::kEarly) mem_sync();
+    if constexpr (kDefer)
+      keep.routed = fb;
+    else if (tid < E)
+      a.routed[tid] = (unsigned char)fb;
+    if constexpr (!Caller::kEarly) lds_sync();
     if constexpr (W > 1) wave_sums<W>(L.wsum[0], wave, before, all);
     distinct = all >> 16;
     total = all & 0xFFFF;
     const int j = (before & 0xFFFF) + __popcll(mask & lanes_below());
     if (m && j < a.max_inserts && distinct <= a.max_distinct) {
       L.mis[j] = tid;
-      a.miss[2 * j] = tid;
+      if constexpr (kDefer)
+        keep.miss = j;
+      else
+        a.miss[2 * j] = tid;
     }
   } else {
     int n = 0;
@@ -330,7 +370,10 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   }
   const long long st = uniform_i64(st_v) + 1;
   if (distinct > a.max_distinct) {  // wide step: read through, nothing else changes
-    if (tid == 0) {
+    if constexpr (kDefer) {
+      keep.step = st;
+      caller.stores = keep;
+    } else if (tid == 0) {
       if constexpr (!PF) a.step[0] = st;
       a.n_miss[0] = 0;
     }
@@ -353,8 +396,12 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
       sp = ageing ? 1 : 0;
       hit = true;
     } else {
-      a.table[se] = -1;
-      a.map_cold[se] = se;
+      if constexpr (kDefer) {
+        keep.dropped = se;
+      } else {
+        a.table[se] = -1;
+        a.map_cold[se] = se;
+      }
       if constexpr (!GLOBAL_E) L.tab[se] = -1;
       se = -1;
       sp = 0;
@@ -494,25 +541,75 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     if constexpr (W == 1) lds_sync();  // L.mis, in the paths above that made no sync
     if (r >= 0) {
       const int e = L.mis[r];
-      if (se >= 0 && se < E) {
-        a.table[se] = -1;
-        a.map_cold[se] = se;
-        if constexpr (!GLOBAL_E) L.tab[se] = -1;
+      const bool evicts = se >= 0 && se < E;
+      if constexpr (kDefer) {
+        if (evicts) keep.evicted = se;
+        keep.insert = r;
+        keep.expert = e;
+        L.vic[r] = tid;
+      } else {
+        if (evicts) {
+          a.table[se] = -1;
+          a.map_cold[se] = se;
+        }
+        a.table[e] = tid;
+        a.map_cold[e] = -1;
+        a.miss[2 * r + 1] = tid;
       }
-      a.table[e] = tid;
-      a.map_cold[e] = -1;
-      a.miss[2 * r + 1] = tid;
-      if constexpr (!GLOBAL_E) L.tab[e] = tid;
+      if constexpr (!GLOBAL_E) {
+        if (evicts) L.tab[se] = -1;
+        L.tab[e] = tid;
+      }
       se = e;
       sp = fresh;
       moved = aged = true;
     }
   }
-  if (slot && aged) a.slot_stamp[tid] = sp;
-  if (slot && moved) a.slot_expert[tid] = se;
+  if constexpr (kDefer) {
+    keep.served = true;
+    keep.inserting = nins > 0;
+    keep.moved = slot && moved;
+    keep.aged = slot && aged;
+    keep.slot_expert = se;
+    keep.slot_stamp = sp;
+    keep.step = st;
+    keep.nact = nact;
+    caller.stores = keep;
+  } else {
+    if (slot && aged) a.slot_stamp[tid] = sp;
+    if (slot && moved) a.slot_expert[tid] = se;
+    if (tid == 0) {
+      if constexpr (!PF) a.step[0] = st;
+      a.n_miss[0] = nact;
+    }
+  }
+}
+
+// A deferred step's stores.
+__device__ __forceinline__ void store_step(const ManageArgs& a, const StepStores& s) {
+  const int tid = threadIdx.x;
+  if (tid < a.E) a.routed[tid] = (unsigned char)s.routed;
+  if (s.served) {
+    if (s.miss >= 0) a.miss[2 * s.miss] = tid;
+    if (s.dropped >= 0) {
+      a.table[s.dropped] = -1;
+      a.map_cold[s.dropped] = s.dropped;
+    }
+    if (s.insert >= 0) {
+      if (s.evicted >= 0) {
+        a.table[s.evicted] = -1;
+        a.map_cold[s.evicted] = s.evicted;
+      }
+      a.table[s.expert] = tid;
+      a.map_cold[s.expert] = -1;
+      a.miss[2 * s.insert + 1] = tid;
+    }
+    if (s.aged) a.slot_stamp[tid] = s.slot_stamp;
+    if (s.moved) a.slot_expert[tid] = s.slot_expert;
+  }
   if (tid == 0) {
-    if constexpr (!PF) a.step[0] = st;
-    a.n_miss[0] = nact;
+    a.step[0] = s.step;
+    a.n_miss[0] = s.nact;
   }
 }
 

@@ -1,12 +1,12 @@
 """ctypes binding of libexpertcache.so (C-ABI in include/expert_cache.h).
 
 Same search order and same argument lists for the reference's two bound entry points
-(vllm_expert_cache/_lib.py:15-61): manage and gather. Six more are bound here:
+(vllm_expert_cache/_lib.py:15-61): manage and gather. Seven more are bound here:
 `expert_cache_fused` (exported by the reference but never bound), the two remap entry
 points that replace the reference's torch remap, `expert_cache_prefetch`,
 `expert_cache_manage_remap_prefetch` (one layer's policy step with another's prefetch step
-in one launch), and `expert_cache_gather_live` (the prefetch copy that stops for dropped
-predictions). Every call is asynchronous on the caller's stream and never reads a device
+in one launch), `expert_cache_gather_live` (the prefetch copy that stops for dropped
+predictions), and `expert_cache_refresh` (policy step, remap and gather in one call). Every call is asynchronous on the caller's stream and never reads a device
 value back, so the whole path is HIP-graph capturable.
 
 There is no fallback: if the library or one of its symbols is missing, loading fails with
@@ -55,7 +55,18 @@ SIGNATURES = {
     #                       pf_miss, pf_n_miss, stream)
     "expert_cache_manage_remap_prefetch": ([_P] + [_I] * 6 + [_P] * 8 + [_I, _I, _P]
                                            + [_P, _I, _I] + [_P] * 7 + [_P]),
+    # refresh(layer, ids, id_bytes, mk, out, stream)
+    "expert_cache_refresh": [_P, _P, _I, _I, _P, _P],
 }
+
+
+class Layer(ctypes.Structure):
+    """expert_cache_layer: what `expert_cache_refresh` needs of one layer."""
+
+    _fields_ = ([(n, _I) for n in ("E", "S", "policy", "decay", "chunks", "lanes")]
+                + [(n, _P) for n in ("table", "map_cold", "slot_expert", "slot_stamp",
+                                     "routed", "step", "miss", "n_miss", "arrived")]
+                + [("dst", _P * 6), ("src", _P * 6), ("bytes", _L * 6)])
 
 
 def library_path() -> str:

@@ -2,13 +2,16 @@
 
 The layer's full expert tensors stay where the offloader put them (host memory the GPU can
 read). This class adds `num_slots` HBM slot buffers per mirrored tensor and the device
-state of the replacement policy. Each served decode step runs, on the current stream:
+state of the replacement policy. Each served decode step runs, on the current stream,
+expert_cache_refresh, which is in one launch
 
   1. expert_cache_manage_remap: marks the routed experts, refreshes their priority, evicts
      the lowest-priority slots this step does not need, installs the missing experts, writes
-     the (expert, slot) miss list, and rewrites the routing ids into slot ids -- one
-     single-wave kernel.
+     the (expert, slot) miss list, and rewrites the routing ids into slot ids;
   2. expert_cache_gather: pulls each missing expert's slabs from host memory into its slot.
+
+Where a prefetch is staged with the step or its copy is still under way, the two are launched
+one after the other.
 
 The fused-MoE GEMM then runs unchanged against the slot buffers with the slot ids. Nothing
 reads a device value back to the host, so the sequence is graph-capturable, and the kernels
@@ -33,7 +36,7 @@ import os
 
 import torch
 
-from ._lib import GATHER_SLOTS, lib
+from ._lib import GATHER_SLOTS, Layer, lib
 from .config import settings
 
 # Gather grid: chunks x lanes workgroups of 256 lanes, each holding one 8-KB tile of loads
@@ -146,6 +149,8 @@ class ExpertSlotCache:
         # step writes `miss`
         self.pf_miss = torch.zeros((2 * self.S,), dtype=i32, device=device)
         self.pf_n_miss = torch.zeros((1,), dtype=i32, device=device)
+        # workgroups of a refresh launch that have read the state (zero between launches)
+        self.arrived = torch.zeros((1,), dtype=i32, device=device)
         self._pf_fork = self._pf_done = None
         self._pf_pending = False
         # prefetch staged to ride with this cache's next policy launch: (cache, ids, budget)
@@ -163,6 +168,7 @@ class ExpertSlotCache:
         self._gather_key = None
         self._gather_srcs = ()
         self._gather_calls = ()
+        self._layer = self._layer_at = None
 
         self.policy = settings.policy_code
         self.decay = settings.decay
@@ -211,6 +217,14 @@ class ExpertSlotCache:
         ids, nbytes = self._id_view(topk_ids)
         out = torch.empty_like(ids)
         mk = int(ids.numel())
+        if self._rider is None and not self._pf_pending and self._layer_at is not None:
+            rc = h.expert_cache_refresh(self._layer_at, ids.data_ptr(), nbytes, mk,
+                                        out.data_ptr(), stream)
+            if rc != 0:
+                raise RuntimeError(f"expert_cache_refresh failed rc={rc}")
+            if len(self._gather_calls) > 1:
+                self._gather(self._gather_calls[1:], self.miss, self.n_miss, stream)
+            return out if out.dtype == topk_ids.dtype else out.to(topk_ids.dtype)
         own = (ids.data_ptr(), nbytes, mk, self.E, self.S, min(self.E, mk), self.S,
                *self._state, self.policy, self.decay, out.data_ptr())
         rider = self._rider
@@ -231,7 +245,7 @@ class ExpertSlotCache:
             rider[0]._copy_prefetched()
         # a prefetched slot may be this step's victim: its copy lands before this gather
         self._wait_copy()
-        self._gather(self.miss, self.n_miss, stream)
+        self._gather(self._gather_calls, self.miss, self.n_miss, stream)
         return out if out.dtype == topk_ids.dtype else out.to(topk_ids.dtype)
 
     def prefetch(self, pred_ids: torch.Tensor, max_inserts: int | None = None,
@@ -311,25 +325,28 @@ class ExpertSlotCache:
         side.wait_event(self._pf_fork)
         # the real step that settles these installs may drop some while this copy runs: the
         # live copy stops loading those
-        self._gather(self.pf_miss, self.pf_n_miss, side.cuda_stream, live=True)
+        self._gather(self._gather_calls, self.pf_miss, self.pf_n_miss, side.cuda_stream,
+                     live=True)
         self._pf_done.record(side)
         self._pf_pending = True
 
     def _plan(self) -> None:
         """Resolve the gather calls against where the sources are now. vLLM's offloader
         may rebind them after the cache is built, so they are re-read every step, and the
-        calls are rebuilt when one moved."""
+        calls are rebuilt when one moved or a launch option changed."""
         srcs = tuple(getattr(self.owner, n).data for n in self.names)
-        key = tuple(t.data_ptr() for t in srcs)
+        key = (self.policy, self.decay, self.chunks, self.lanes,
+               *[t.data_ptr() for t in srcs])
         if key != self._gather_key:
             self._gather_calls = self._gather_plan(srcs)
+            self._layer, self._layer_at = self._layer_plan()
             # holding the sources keeps their addresses from being reused by new tensors
             self._gather_srcs, self._gather_key = srcs, key
 
-    def _gather(self, miss: torch.Tensor, n_miss: torch.Tensor, stream,
+    def _gather(self, calls, miss: torch.Tensor, n_miss: torch.Tensor, stream,
                 live: bool = False) -> None:
-        """expert_cache_gather of every mirrored tensor over one miss list, six per call,
-        with the calls `_plan` resolved; with `live`, expert_cache_gather_live (a prefetch
+        """expert_cache_gather of the tensors of `calls` over one miss list, six per call,
+        as `_plan` resolved them; with `live`, expert_cache_gather_live (a prefetch
         step's list, whose dropped predictions stop copying)."""
         h = lib()
         if live:
@@ -339,10 +356,22 @@ class ExpertSlotCache:
         else:
             fn, name = h.expert_cache_gather, "expert_cache_gather"
             tail = (miss.data_ptr(), n_miss.data_ptr(), self.chunks, self.lanes, stream)
-        for args in self._gather_calls:
+        for args in calls:
             rc = fn(*args, *tail)
             if rc != 0:
                 raise RuntimeError(f"{name} failed rc={rc}")
+
+    def _layer_plan(self):
+        """The layer as expert_cache_refresh takes it, with the first six tensors, and its
+        address; None when no tensor is mirrored."""
+        if not self._gather_calls:
+            return None, None
+        first = self._gather_calls[0]
+        trio = ctypes.c_void_p * GATHER_SLOTS
+        layer = Layer(self.E, self.S, self.policy, self.decay, self.chunks, self.lanes,
+                      *self._state, self.arrived.data_ptr(), trio(*first[0::3]),
+                      trio(*first[1::3]), (ctypes.c_long * GATHER_SLOTS)(*first[2::3]))
+        return layer, ctypes.addressof(layer)
 
     def _gather_plan(self, srcs) -> tuple:
         """The (dst, src, bytes) x 6 argument lists of the gather calls, padded with a
