@@ -34,11 +34,12 @@ __device__ __forceinline__ void put_row(unsigned long long* row, unsigned long l
 
 // manage_k<W, GLOBAL_E, 4, true> with stamps
 template <int W, bool GLOBAL_E>
-__global__ __launch_bounds__(W* kWave) void stamped_manage_k(ManageArgs a,
+__global__ __launch_bounds__(W* kWave) void stamped_manage_k(EC_STEP_PARAMS, ManageArgs rest,
                                                              unsigned long long* row) {
   const unsigned long long t0 = clock_now();
   __shared__ ManageLds<W, GLOBAL_E> L;
-  args_in_sgprs(a);
+  const ManageArgs a =
+      step_args(ids, step, slot_expert, slot_stamp, table, mk, E, S, rest);
   long long idv;
   manage_step<W, GLOBAL_E, 4>(a, L, idv);
   step_sync<GLOBAL_E>();
@@ -69,7 +70,8 @@ __global__ __launch_bounds__(kWave) void stamped_empty_k(unsigned long long* row
 
 template <int W, bool GLOBAL_E = false>
 void launch_waves(const ManageArgs& a, unsigned long long* row, hipStream_t s) {
-  hipLaunchKernelGGL((stamped_manage_k<W, GLOBAL_E>), dim3(1), dim3(W * kWave), 0, s, a, row);
+  hipLaunchKernelGGL((stamped_manage_k<W, GLOBAL_E>), dim3(1), dim3(W * kWave), 0, s,
+                     EC_STEP_ARGS(a), a, row);
 }
 
 }  // namespace

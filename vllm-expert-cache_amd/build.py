@@ -27,6 +27,8 @@ ARCH = os.environ.get("EXPERT_CACHE_ARCH", "gfx950")
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
              # keep hipcc from emitting packed-FP32 instructions (v_pk_*_f32)
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+             # leading scalar kernel arguments arrive in SGPRs (14 words is the most)
+             "-mllvm", "-amdgpu-kernarg-preload-count=14",
              "-Wall"]
 
 

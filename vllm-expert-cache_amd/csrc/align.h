@@ -261,13 +261,17 @@ __device__ __forceinline__ AlignTotals align_place_wave(const AlignArgs& g, int 
 // loads are in flight (the step's second sync waits for those stores); the ids and the
 // blocks' experts are then stored over them, so padding needs no pass of its own.
 template <int W>
-__global__ __launch_bounds__(W* kWave) void fused_k(ManageArgs a, AlignArgs g) {
+__global__ __launch_bounds__(W* kWave) void fused_k(EC_STEP_PARAMS, ManageArgs rest, AlignArgs g) {
   constexpr int T = W * kWave;
   __shared__ ManageLds<W, false> L;
   __shared__ AlignLds<W> A;
-  args_in_sgprs(a);
+  const ManageArgs a =
+      step_args(ids, step, slot_expert, slot_stamp, table, mk, E, S, rest);
   const int tid = threadIdx.x;
-  const int E = a.E, S = a.S, mk = a.mk, waves = (mk + kWave - 1) / kWave;
+  const int waves = (mk + kWave - 1) / kWave;
+  // the alignments' arguments arrive with the step's
+  asm volatile("" ::"s"(g.sorted_hot), "s"(g.sorted_cold), "s"(g.eids_hot), "s"(g.eids_cold),
+               "s"(g.L), "s"(g.NB), "s"(g.bs), "s"(g.div_mul), "s"(g.div_shift));
   const BlockDiv d(g);
   long long idv;
   const auto early = [&] {
@@ -361,14 +365,16 @@ __global__ __launch_bounds__(1024) void align_k(const int* ids, int mk, int E, i
 
 // The policy step in the launch's first workgroup; the others store the alignments' defaults.
 template <int W>
-__global__ __launch_bounds__(W* kWave) void manage_defaults_k(ManageArgs a, AlignArgs g) {
+__global__ __launch_bounds__(W* kWave) void manage_defaults_k(EC_STEP_PARAMS, ManageArgs rest,
+                                                               AlignArgs g) {
   __shared__ ManageLds<W, false> L;
+  const ManageArgs a =
+      step_args(ids, step, slot_expert, slot_stamp, table, mk, E, S, rest);
   if (blockIdx.x > 0) {
     align_defaults(g, a.mk, (blockIdx.x - 1) * W * kWave + threadIdx.x,
                    (gridDim.x - 1) * W * kWave);
     return;
   }
-  args_in_sgprs(a);
   long long idv;
   manage_step<W, false, 4>(a, L, idv);
 }

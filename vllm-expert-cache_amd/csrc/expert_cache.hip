@@ -58,11 +58,11 @@ template <int IDB, bool REMAP>
 int launch_manage(const ManageArgs& a, hipStream_t stream) {
   if (a.E > kLdsExperts) {
     hipLaunchKernelGGL((manage_k<16, true, IDB, REMAP>), dim3(1), dim3(16 * kWave), 0, stream,
-                       a);
+                       EC_STEP_ARGS(a), a);
   } else {
     with_waves(waves_for(a.E, a.S, a.mk), [&](auto w) {
       hipLaunchKernelGGL((manage_k<w(), false, IDB, REMAP>), dim3(1), dim3(w() * kWave), 0,
-                         stream, a);
+                         stream, EC_STEP_ARGS(a), a);
     });
   }
   return (int)hipGetLastError();
@@ -97,7 +97,8 @@ int launch_manage_prefetch(const ManageArgs& a, const ManageArgs& p, hipStream_t
 int launch_fused(const ManageArgs& a, const AlignArgs& g, hipStream_t stream) {
   if (a.mk <= kFusedIds) {
     with_waves(waves_for(a.E, a.S, 4 * a.mk), [&](auto w) {
-      hipLaunchKernelGGL((fused_k<w()>), dim3(1), dim3(w() * kWave), 0, stream, a, g);
+      hipLaunchKernelGGL((fused_k<w()>), dim3(1), dim3(w() * kWave), 0, stream,
+                         EC_STEP_ARGS(a), a, g);
     });
     return (int)hipGetLastError();
   }
@@ -105,7 +106,7 @@ int launch_fused(const ManageArgs& a, const AlignArgs& g, hipStream_t stream) {
   const int fills = g.L / 16384 < 255 ? g.L / 16384 + 1 : 256;
   with_waves(waves_for(a.E, a.S, a.mk), [&](auto w) {
     hipLaunchKernelGGL((manage_defaults_k<w()>), dim3(1 + fills), dim3(w() * kWave), 0, stream,
-                       a, g);
+                       EC_STEP_ARGS(a), a, g);
   });
   const int rc = (int)hipGetLastError();
   if (rc) return rc;
@@ -264,9 +265,11 @@ int expert_cache_refresh(const expert_cache_layer* c, const void* ids, int id_by
   const dim3 grid(c->chunks, c->lanes), block(kGatherThreads);
   if (c->E <= kGatherThreads && c->S <= kGatherThreads) {
     if (id_bytes == 8)
-      hipLaunchKernelGGL((refresh_k<8>), grid, block, 0, stream, a, g, c->arrived);
+      hipLaunchKernelGGL((refresh_k<8>), grid, block, 0, stream, EC_STEP_ARGS(a), a, g,
+                         c->arrived);
     else
-      hipLaunchKernelGGL((refresh_k<4>), grid, block, 0, stream, a, g, c->arrived);
+      hipLaunchKernelGGL((refresh_k<4>), grid, block, 0, stream, EC_STEP_ARGS(a), a, g,
+                         c->arrived);
     return (int)hipGetLastError();
   }
   const int rc = id_bytes == 8 ? launch_manage<8, true>(a, stream)

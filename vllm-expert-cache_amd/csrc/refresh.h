@@ -28,12 +28,13 @@ namespace ec {
 constexpr int kRefreshWaves = kGatherThreads / kWave;
 
 template <int IDB>
-__global__ __launch_bounds__(kGatherThreads) void refresh_k(ManageArgs a, GatherArgs g,
-                                                            unsigned* arrived) {
+__global__ __launch_bounds__(kGatherThreads) void refresh_k(EC_STEP_PARAMS, ManageArgs rest,
+                                                            GatherArgs g, unsigned* arrived) {
   constexpr int W = kRefreshWaves;
   __shared__ ManageLds<W, false> L;
   __shared__ int last;
-  args_in_sgprs(a);
+  const ManageArgs a =
+      step_args(ids, step, slot_expert, slot_stamp, table, mk, E, S, rest);
   StepStores stores;
   long long idv;
   manage_step<W, false, IDB>(a, L, idv, DeferredStep(stores));
