@@ -255,7 +255,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const int e = (int)idv;
     if (e >= 0 && e < E) flag[e] = 1;
   }
-  if (mk > T) {
+  if (__builtin_expect(mk > T, 0)) {
     const auto mark = [&](int e) {
       if (e >= 0 && e < E) flag[e] = 1;
     };
@@ -369,7 +369,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     }
   }
   const long long st = uniform_i64(st_v) + 1;
-  if (distinct > a.max_distinct) {  // wide step: read through, nothing else changes
+  if (__builtin_expect(distinct > a.max_distinct, 0)) {  // wide step: read through, nothing else changes
     if constexpr (kDefer) {
       keep.step = st;
       caller.stores = keep;
@@ -388,7 +388,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   bool hit = !PF && slot && L.hit[tid] != 0;
   bool moved = false;  // slot_expert[tid] changes
   bool aged = false;   // slot_stamp[tid] changes
-  if (!PF && held && sp < 0) {
+  if (__builtin_expect(!PF && held && sp < 0, 0)) {
     // A routed one is handed to the hit refresh below at the stamp that makes it end the
     // step at an install's stamp: 0 (+1 = 1 under LFU; st under LRU), or 1 when this step
     // ages (+1, halved = 1). Distinct slots hold distinct experts: no write conflicts.
@@ -437,8 +437,8 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const bool few = nins <= few_inserts<W>(S);
     int r = -1;  // insert this thread's slot takes
     if constexpr (W > 1) {
-      // waves without slots have nothing to sort
-      const unsigned sorted = few || wave * kWave >= S ? key : wave_sort(key);
+      // a wave without an evictable slot has nothing to sort
+      const unsigned sorted = few || (nev_wave & 0xFFFF) == 0 ? key : wave_sort(key);
       L.key[tid] = sorted;
       L.ins[tid] = -1;
       if (lane == 0) L.wev[wave] = nev_wave;
@@ -446,7 +446,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
       int before;
       wave_sums<W>(L.wev, wave, before, nev);
       nact = min(nins, nev & 0xFFFF);
-      if (nev <= 0xFFFF && nact <= kWave) {
+      if (__builtin_expect(nev <= 0xFFFF && nact <= kWave, 1)) {
         if (wave == 0) {
           unsigned v = sorted;  // to become, in lane i, the i-th smallest key
           if (few) {
@@ -523,7 +523,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
         }
       }
     }
-    if (nev > 0xFFFF) {
+    if (__builtin_expect(nev > 0xFFFF, 0)) {
       // stamps too far apart for 32-bit keys: rank by counting on the 64-bit ones
       const long long k64 = ev ? victim_key(sp, tid) : kKeyMax;
       L.key64[tid] = k64;
