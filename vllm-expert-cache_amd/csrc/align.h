@@ -201,7 +201,7 @@ __device__ __forceinline__ AlignTotals align_place(const AlignArgs& g, AlignLds<
       const bool many = own && q1 - q0 > 8;
       if (own && !many)
         for (int q = q0; q < q1; ++q) eids[q] = tid;
-      for (unsigned long long m = __ballot(many); m != 0; m &= m - 1) {
+      for (unsigned long long m = ballot(many); m != 0; m &= m - 1) {
         const int l = __ffsll((long long)m) - 1;
         const int end = __builtin_amdgcn_readlane(q1, l);
         for (int q = __builtin_amdgcn_readlane(q0, l) + lane; q < end; q += kWave)
@@ -229,16 +229,16 @@ __device__ __forceinline__ AlignTotals align_place_wave(const AlignArgs& g, int 
   const int b = (int)(s >> 6);
   const bool valid = s != none;
   const int prev = __builtin_amdgcn_update_dpp(-1, b, 0x138, 0xF, 0xF, false);  // lane - 1's
-  const unsigned long long heads = __ballot(valid & (b != prev));
+  const unsigned long long heads = ballot(valid & (b != prev));
   const unsigned long long upto = lanes_below() << 1 | 1ull;  // this lane and those below
   const int head = 63 - __clzll((long long)(heads & upto));
   const unsigned long long later = heads & ~upto;
-  const int nvalid = (int)__popcll(__ballot(valid));
+  const int nvalid = (int)__popcll(ballot(valid));
   const int next = later ? __ffsll((long long)later) - 1 : nvalid;
   const int padded = d.pad(next - head);
   const bool first = valid & (b != prev);
   const int scan = wave_incl_scan(first ? padded : 0);
-  const int nhot = (int)__popcll(__ballot(valid & (b < S)));
+  const int nhot = (int)__popcll(ballot(valid & (b < S)));
   const int all = __builtin_amdgcn_readlane(scan, kWave - 1);
   const int at = __builtin_amdgcn_readlane(scan, max(nhot - 1, 0));
   const int hot = nhot > 0 ? at : 0;

@@ -142,6 +142,13 @@ __device__ __forceinline__ long long uniform_i64(long long v) {
   return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
+// Makes the kernel arguments that the step needs late live in SGPRs at this point, so that
+// the compiler loads them together, instead of each where it is used, behind a wait.
+__device__ __forceinline__ void args_in_sgprs(const ManageArgs& a) {
+  asm volatile("" ::"s"(a.map_cold), "s"(a.routed), "s"(a.miss), "s"(a.n_miss), "s"(a.out),
+               "s"(a.max_distinct), "s"(a.max_inserts), "s"(a.policy), "s"(a.decay));
+}
+
 // What one thread (expert `tid`, slot `tid`) has to store for a step. A kernel whose
 // workgroups all run the step has one of them store it, once all have read the state.
 struct StepStores {
@@ -245,6 +252,10 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   }
   if (tid < T / 4) reinterpret_cast<unsigned*>(L.hit)[tid] = 0;
   step_sync<GLOBAL_E>();
+  // while the loads above are in flight; where `early` ran, its own arguments came first, and
+  // waiting for these here measured slower (8 fused ids 140.5 -> 142.0 us for 48 launches,
+  // against 99.8 -> 98.1 for the policy step alone)
+  if constexpr (!Caller::kEarly) args_in_sgprs(a);
 
   // ---- routed flags (ids outside [0,E) are padding; int64 ids truncate like .to(int32))
   // The sentinels for threads past mk / S are applied only now, after the first fence, so
@@ -302,9 +313,9 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const int fb = flag[tid];  // zero past E
     const bool m = (fb != 0) & (tv < 0);
     if (!PF && fb != 0 && tv >= 0 && tv < S) L.hit[tv] = 1;
-    const unsigned long long mask = __ballot(m);
+    const unsigned long long mask = ballot(m);
     // both counts in one word: neither exceeds 1024 over the workgroup
-    const int mine = (int)(__popcll(__ballot(fb != 0)) << 16 | __popcll(mask));
+    const int mine = (int)(__popcll(ballot(fb != 0)) << 16 | __popcll(mask));
     int before = 0, all = mine;
     if constexpr (PF) {
       // the prefetch step has no step counter to measure stamps from: their maximum serves
@@ -354,7 +365,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
         const int t = f ? a.table[e] : -1;
         if (!PF && f && t >= 0 && t < S) L.hit[t] = 1;
         const bool m = f && t < 0;
-        const unsigned long long mask = __ballot(m);
+        const unsigned long long mask = ballot(m);
         if (lane == 0) L.wsum[buf][wave] = __popcll(mask);
         lds_sync();
         int all;
@@ -432,7 +443,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     bool fits;
     unsigned key = victim_key32<SB>(sp, base, tid, fits);
     if (!ev) key = kKeyNone;
-    const int nev_wave = (int)__popcll(__ballot(ev)) | (__ballot(ev & !fits) ? 1 << 16 : 0);
+    const int nev_wave = (int)__popcll(ballot(ev)) | (ballot(ev & !fits) ? 1 << 16 : 0);
     int nev = nev_wave;
     const bool few = nins <= few_inserts<W>(S);
     int r = -1;  // insert this thread's slot takes
@@ -632,15 +643,6 @@ __device__ __forceinline__ void remap_tail(const ManageArgs& a,
     store_id<IDB>(a.out, i, lookup(load_id<IDB>(a.ids, i)));
 }
 
-// Makes every kernel argument live in SGPRs at this point, so the compiler issues all the
-// argument loads together (one round trip) instead of sinking some into later branches.
-__device__ __forceinline__ void args_in_sgprs(const ManageArgs& a) {
-  asm volatile("" ::"s"(a.ids), "s"(a.table), "s"(a.map_cold), "s"(a.slot_expert),
-               "s"(a.slot_stamp), "s"(a.routed), "s"(a.step), "s"(a.miss), "s"(a.n_miss),
-               "s"(a.out), "s"(a.mk), "s"(a.E), "s"(a.S), "s"(a.max_distinct),
-               "s"(a.max_inserts), "s"(a.policy), "s"(a.decay));
-}
-
 // What the step's first loads need are a kernel's first arguments, outside the struct: the
 // build has the command processor preload up to 14 words of leading scalar arguments into
 // SGPRs, so those loads wait for no argument load (a struct is not preloaded); the struct's
@@ -683,7 +685,6 @@ __global__ __launch_bounds__(W* kWave) void manage_k(EC_STEP_PARAMS, ManageArgs 
 template <int W, bool GLOBAL_E>
 __global__ __launch_bounds__(W* kWave) void prefetch_k(ManageArgs a) {
   __shared__ ManageLds<W, GLOBAL_E> L;
-  args_in_sgprs(a);
   long long idv;
   manage_step<W, GLOBAL_E, 4, true>(a, L, idv);
 }
@@ -697,12 +698,10 @@ __global__ __launch_bounds__(W* kWave) void manage_prefetch_k(ManageArgs a, Mana
   __shared__ ManageLds<W, GLOBAL_E> L;
   long long idv;
   if (blockIdx.x == 0) {
-    args_in_sgprs(a);
     manage_step<W, GLOBAL_E, IDB>(a, L, idv);
     step_sync<GLOBAL_E>();
     remap_tail<W, GLOBAL_E, IDB>(a, L, idv);
   } else {
-    args_in_sgprs(p);
     manage_step<W, GLOBAL_E, 4, true>(p, L, idv);
   }
 }

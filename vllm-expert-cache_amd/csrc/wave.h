@@ -26,6 +26,11 @@ __device__ __forceinline__ void mem_sync() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 }
 
+// The lanes where `p` holds (HIP's __ballot takes an int: two more instructions).
+__device__ __forceinline__ unsigned long long ballot(bool p) {
+  return __builtin_amdgcn_ballot_w64(p);
+}
+
 __device__ __forceinline__ unsigned long long lanes_below() {
   return (1ull << __lane_id()) - 1ull;
 }
@@ -176,14 +181,14 @@ __device__ __forceinline__ unsigned wave_merge_low(unsigned v, unsigned down) {
 // bits (all lanes must be active). One ballot per bit: needs no LDS, and no order among the
 // lanes is assumed.
 __device__ __forceinline__ unsigned long long wave_match(int v, int bits) {
-  const unsigned long long valid = __ballot(v >= 0);
+  const unsigned long long valid = ballot(v >= 0);
   unsigned lo = (unsigned)valid, hi = (unsigned)(valid >> 32);
 #pragma unroll 1
   for (int b = 0; b < bits; b += 3) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int bit = __builtin_amdgcn_sbfe(v, b + k, 1);  // 0 or -1
-      const unsigned long long set = __ballot(bit != 0);
+      const unsigned long long set = ballot(bit != 0);
       lo &= ~((unsigned)set ^ (unsigned)bit);
       hi &= ~((unsigned)(set >> 32) ^ (unsigned)bit);
     }
