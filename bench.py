@@ -709,7 +709,7 @@ def main():
                      "achieved_events": round(tw["achieved"], 3),
                      "frac_events": round(tw["achieved"] / peak, 4),
                      # the metric's other two parts, as scalars beside the gather's
-                     "policy_kernel": "manage_k (policy step + fused remap, one wavefront)",
+                     "policy_kernel": "manage_k (policy step + fused remap, one workgroup)",
                      "policy_bound": "latency",
                      "policy_us_per_layer": manage_us,
                      "policy_kernel_us_in_chain":
@@ -1388,7 +1388,7 @@ def fused_leg(torch, np, lib, dev, hold):
                      "inserts_per_layer_step": round(inserts, 4)})
         log(f"fused {name}: E={E} S={S} mk={mk} bs={FUSED_BS}, {us:.2f} us/layer-step in "
             f"graph replay, {int(policy_bytes + out_bytes)} algorithmic bytes per call")
-    return {"bound": "latency (one wave, dependent LDS phases)", "layers": FUSED_LAYERS,
+    return {"bound": "latency (one workgroup, dependent LDS phases)", "layers": FUSED_LAYERS,
             "steps": FUSED_STEPS, "def": "graph replay of one launch per layer, including "
             "the per-step id copy, steps queued in chunks behind stream holds so the host's "
             "launch rate is out of the figure; LRU, cold start. cpu_baseline.fused_us_per_layer_step is "

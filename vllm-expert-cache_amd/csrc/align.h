@@ -22,8 +22,8 @@
 //    which costs less than the node or the cross-XCD handoff that sharing the counts would.
 //
 // Measured on MI355X, us a launch in a graph, against the same work in one wave that staged
-// its output in LDS: 8 ids (128 experts, 64 slots, block 16) 4.7 -> 3.9; 512 ids (256, 128,
-// 16) 12.6 -> 7.3; 16384 ids (128, 64, 64) 232 -> 15.6.
+// its output in LDS: 8 ids (128 experts, 64 slots, block 16) 4.7 -> 2.9; 512 ids (256, 128,
+// 16) 12.5 -> 5.3; 16384 ids (128, 64, 64) 232 -> 12.3; 65536 ids 800 -> 18.
 #pragma once
 #include "manage.h"
 

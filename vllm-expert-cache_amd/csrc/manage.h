@@ -5,9 +5,8 @@
 //
 //  * The workgroup has W waves, as many as give every expert and every slot a thread of its
 //    own (64 W >= E and S; above 1024 experts 16 waves walk the experts). What bounds the
-//    step is latency, and a large part of it is instruction fetch: a launch finds its code
-//    in no cache of the XCD it lands on. With one element a thread every phase is one short
-//    piece of straight code, whatever E and S.
+//    step is latency, and the instructions a wave runs through are a large part of it. With
+//    one element a thread every phase is one short piece of straight code, whatever E and S.
 //  * Every global load the step needs (step counter, ids, slot_expert, slot_stamp, table) is
 //    issued up front, so the step costs one memory round trip plus the stores. Cross-lane
 //    traffic is DPP and ballots, cross-wave traffic LDS behind barriers that wait for LDS
@@ -25,8 +24,8 @@
 //    keys by counting.
 //
 // Measured on MI355X, us for a graph of 48 launches, against a one-wave kernel that held up to
-// 16 slots and 8 experts a lane: 128 experts, 64 slots, 8 ids 111 -> 104; 256, 192, 128 ids,
-// 6.6 inserts a launch 246 -> 159; 512, 257, 50 ids, 2.6 inserts 274 -> 153.
+// 16 slots and 8 experts a lane: 128 experts, 64 slots, 8 ids 111 -> 99; 256, 192, 128 ids,
+// 6.6 inserts a launch 246 -> 151; 512, 257, 50 ids, 2.6 inserts 274 -> 146.
 #pragma once
 #include <type_traits>
 

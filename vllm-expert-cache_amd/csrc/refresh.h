@@ -15,9 +15,10 @@
 //    Counting at every step, before it is known whether it inserts, put the ticket's round
 //    trip (over a microsecond) into the steps that insert nothing and gained nothing.
 //
-// Measured on MI355X, us for a graph of 32 layer-steps, against the two launches: 128 experts
-// of 4.7 MB, 96 slots, 8 ids, 0.2 inserts a step 404 -> 373; 64 slots, 0.5 inserts 1350 ->
-// 1318 (the host link's time is 1230). Four refreshes called from Python 64 -> 47.
+// Measured on MI355X, us for a graph of 32 layer-steps, against the two launches of a one-wave
+// step and the gather: 128 experts of 4.7 MB, 8 ids, 96 slots, 0.1 inserts a step 422 -> 374;
+// 64 slots, 0.45 inserts 1334 -> 1290 (the host link's time is 1172). Four refreshes called
+// from Python 65 -> 47.
 #pragma once
 #include "gather.h"
 #include "manage.h"
