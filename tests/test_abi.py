@@ -8,8 +8,11 @@ with the same verdicts as the reference library compiled from its own source
 from __future__ import annotations
 
 import ctypes
+import json
 import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -77,7 +80,6 @@ def test_header_compiles_as_c_and_links(tmp_path):
     """A plain C11 caller (gcc, no HIP headers) compiles against include/expert_cache.h with
     every warning an error, links against the library, and gets -1 from each refused call."""
     import shutil
-    import subprocess
 
     gcc = shutil.which("gcc")
     if gcc is None:
@@ -277,3 +279,80 @@ def test_refresh_refuses_what_its_two_calls_refuse(lib):
     assert call(layer(), id_bytes=2) == -1
     assert call(layer(), mk=-1) == -1
     assert call(layer(), out=None) == -1
+
+
+_RECORDER = r"""
+/* stands before libamdhip64 in the symbol search: kernel launches are recorded, not made */
+typedef struct { unsigned x, y, z; } dim3;
+int launches, groups[8], threads[8];
+static dim3 grid_, block_;
+int __hipPushCallConfiguration(dim3 grid, dim3 block, unsigned long lds, void* stream) {
+  (void)lds; (void)stream;
+  grid_ = grid;
+  block_ = block;
+  return 0;
+}
+int __hipPopCallConfiguration(dim3* grid, dim3* block, unsigned long* lds, void** stream) {
+  *grid = grid_;
+  *block = block_;
+  *lds = 0;
+  *stream = 0;
+  return 0;
+}
+int hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, unsigned long lds,
+                    void* stream) {
+  (void)f; (void)args; (void)lds; (void)stream;
+  groups[launches & 7] = grid.x * grid.y * grid.z;
+  threads[launches++ & 7] = block.x;
+  return 0;
+}
+int hipGetLastError(void) { return 0; }
+"""
+
+_RECORD = """
+import ctypes, json, sys
+rec = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+from vllm_expert_cache import _lib
+lib, out = _lib.lib(), []
+def ints(name):
+    return (ctypes.c_int * 8).in_dll(rec, name)
+for case in json.loads(sys.argv[2]):
+    f = {n: 4096 for n, _ in _lib.Layer._fields_}
+    f.update(policy=1, decay=64, bytes=16, **case["layer"])
+    for n, t in (("dst", ctypes.c_void_p), ("src", ctypes.c_void_p), ("bytes", ctypes.c_long)):
+        f[n] = (t * 6)(*[f[n]] * 6)
+    layer = _lib.Layer(**f)
+    ctypes.c_int.in_dll(rec, "launches").value = 0
+    rc = lib.expert_cache_refresh(ctypes.addressof(layer), case["ids"], case["id_bytes"],
+                                  case["mk"], case["out"], None)
+    assert rc == 0, rc
+    n = ctypes.c_int.in_dll(rec, "launches").value
+    out.append(list(zip(ints("groups")[:n], ints("threads")[:n])))
+print(json.dumps(out))
+"""
+
+
+def _refresh_launches(tmp_path, cases):
+    """[(workgroups, threads) of every launch] that expert_cache_refresh would make for each
+    case, in a child process with a recorder in the HIP launch's place."""
+    src, so = tmp_path / "recorder.c", tmp_path / "recorder.so"
+    src.write_text(_RECORDER)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", str(src), "-o", str(so)], check=True)
+    full = [dict({"ids": 1 << 20, "out": 1 << 21, "id_bytes": 4, "mk": 8}, **c,
+                 layer=dict({"E": 128, "S": 64, "chunks": 32, "lanes": 1}, **c.get("layer", {})))
+            for c in cases]
+    env = dict(os.environ, PYTHONPATH=str(Path(_lib.__file__).resolve().parent.parent))
+    res = subprocess.run([sys.executable, "-c", _RECORD, str(so), json.dumps(full)], env=env,
+                         check=True, capture_output=True, text=True)
+    return [[tuple(x) for x in launches] for launches in json.loads(res.stdout)]
+
+
+def test_refresh_in_place_takes_two_launches(tmp_path):
+    """The one launch's first workgroup may write `out` while the others read `ids`: where the
+    two share a byte, the policy step runs in one workgroup and the gather after it."""
+    at = 1 << 20
+    apart = [{"out": at + 32}, {"out": at - 32}, {"out": at + 64, "id_bytes": 8}]
+    shared = [{"out": at}, {"out": at + 28}, {"out": at - 28}, {"out": at + 60, "id_bytes": 8}]
+    got = _refresh_launches(tmp_path, apart + shared)
+    assert got[:len(apart)] == [[(32, 256)]] * len(apart)
+    assert got[len(apart):] == [[(1, 128), (32, 256)]] * len(shared)

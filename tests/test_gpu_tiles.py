@@ -185,3 +185,31 @@ def test_refresh_in_a_graph():
             for f in ("table", "slot_expert", "slot_stamp", "step", "n_miss"):
                 assert torch.equal(getattr(caches[l], f), getattr(caches[l + 2], f)), (t, l, f)
             assert torch.equal(caches[l].slots["w"], caches[l + 2].slots["w"]), (t, l)
+
+
+@pytest.mark.parametrize("id64", [False, True])
+def test_refresh_in_place(id64):
+    """Slot ids written over the routing ids, beside a twin that gets a buffer of its own."""
+    from types import SimpleNamespace
+
+    from vllm_expert_cache.cache import ExpertSlotCache
+
+    E, S, k = 128, 48, 24
+    rng = np.random.default_rng(5)
+    owner = SimpleNamespace(w=gu.pinned(E * 8208).view(E, 8208))
+    gu.fill_random(owner.w.view(-1), 2)
+    one, two = (ExpertSlotCache(owner, ["w"], E, S, gu.DEV) for _ in range(2))
+    for c in (one, two):
+        c.slots["w"].zero_()
+    one._plan()
+    for t in range(12):
+        ids = torch.as_tensor(rng.integers(-1, E, size=k if t % 3 else 4), device=gu.DEV)
+        ids = ids.to(torch.int64 if id64 else torch.int32)
+        want = two.refresh(ids)
+        assert gu.lib().expert_cache_refresh(one._layer_at, ids.data_ptr(), ids.element_size(),
+                                             ids.numel(), ids.data_ptr(), gu.stream()) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want) and int(one.arrived) == 0, t
+        for f in ("table", "slot_expert", "slot_stamp", "routed", "step", "miss", "n_miss"):
+            assert torch.equal(getattr(one, f), getattr(two, f)), (t, f)
+        assert torch.equal(one.slots["w"], two.slots["w"]), t

@@ -263,7 +263,11 @@ int expert_cache_refresh(const expert_cache_layer* c, const void* ids, int id_by
                                  c->map_cold, c->slot_expert, c->slot_stamp, c->routed, c->step,
                                  c->miss, c->n_miss, c->policy, c->decay, out);
   const dim3 grid(c->chunks, c->lanes), block(kGatherThreads);
-  if (c->E <= kGatherThreads && c->S <= kGatherThreads) {
+  // Of one launch's workgroups the first may write `out` while others still read `ids`, so
+  // ids that are rewritten in place take two launches.
+  const long long id_range = (long long)mk * id_bytes;
+  if (c->E <= kGatherThreads && c->S <= kGatherThreads &&
+      !ranges_meet(ids, id_range, out, id_range)) {
     if (id_bytes == 8)
       hipLaunchKernelGGL((refresh_k<8>), grid, block, 0, stream, EC_STEP_ARGS(a), a, g,
                          c->arrived);
