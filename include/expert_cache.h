@@ -205,9 +205,10 @@ typedef struct expert_cache_layer {
 /*
  * A decode step of one layer: expert_cache_manage_remap with max_distinct = min(E, mk) and
  * max_inserts = S, followed by expert_cache_gather of its miss list, with the same results as
- * the two calls: in one launch where E and S are at most 256 and `out` shares no byte with
- * `ids`, in two otherwise. `layer` is read during the call only. Argument checks are those of
- * the two calls, plus mk >= 0 and `arrived` non-null; nothing runs if one of them fails.
+ * the two calls: in one launch where E and S are at most 256, chunks x lanes at most 128 and
+ * `out` shares no byte with `ids`, in two otherwise. `layer` is read during the call only.
+ * Argument checks are those of the two calls, plus mk >= 0 and `arrived` non-null; nothing
+ * runs if one of them fails.
  *
  * Replaces: vllm_expert_cache/cache.py:112-163; no counterpart in the reference's C-ABI.
  */

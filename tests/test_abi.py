@@ -338,8 +338,8 @@ def _refresh_launches(tmp_path, cases):
     src, so = tmp_path / "recorder.c", tmp_path / "recorder.so"
     src.write_text(_RECORDER)
     subprocess.run(["gcc", "-shared", "-fPIC", "-O1", str(src), "-o", str(so)], check=True)
-    full = [dict({"ids": 1 << 20, "out": 1 << 21, "id_bytes": 4, "mk": 8}, **c,
-                 layer=dict({"E": 128, "S": 64, "chunks": 32, "lanes": 1}, **c.get("layer", {})))
+    full = [{"ids": 1 << 20, "out": 1 << 21, "id_bytes": 4, "mk": 8, **c,
+             "layer": {"E": 128, "S": 64, "chunks": 32, "lanes": 1, **c.get("layer", {})}}
             for c in cases]
     env = dict(os.environ, PYTHONPATH=str(Path(_lib.__file__).resolve().parent.parent))
     res = subprocess.run([sys.executable, "-c", _RECORD, str(so), json.dumps(full)], env=env,
@@ -356,3 +356,17 @@ def test_refresh_in_place_takes_two_launches(tmp_path):
     got = _refresh_launches(tmp_path, apart + shared)
     assert got[:len(apart)] == [[(32, 256)]] * len(apart)
     assert got[len(apart):] == [[(1, 128), (32, 256)]] * len(shared)
+
+
+def test_refresh_takes_two_launches_on_a_large_grid(tmp_path):
+    """Above 128 workgroups the arrivals cost more than a launch saves."""
+    grids = [(128, 1), (16, 8), (1, 1), (129, 1), (16, 64), (1 << 20, 1 << 11)]
+    got = _refresh_launches(tmp_path, [{"layer": {"chunks": c, "lanes": l}} for c, l in grids])
+    assert got[:3] == [[(c * l, 256)] for c, l in grids[:3]]
+    assert got[3:5] == [[(1, 128), (c * l, 256)] for c, l in grids[3:5]]
+    assert len(got[5]) == 2
+
+
+@pytest.mark.parametrize("E,S,launches", [(256, 256, 1), (257, 100, 2), (100, 257, 2)])
+def test_refresh_launches_by_size(tmp_path, E, S, launches):
+    assert len(_refresh_launches(tmp_path, [{"layer": {"E": E, "S": S}}])[0]) == launches

@@ -110,12 +110,12 @@ def test_fused_at_the_workgroups_edges(mk, E, S, bs):
 
 
 @pytest.mark.parametrize("E,S", [(8, 4), (64, 64), (200, 130), (256, 256), (257, 100)])
-@pytest.mark.parametrize("chunks", [1, 7, 32, 300])
+@pytest.mark.parametrize("chunks", [1, 7, 32, 128, 300])
 @pytest.mark.parametrize("id64", [False, True])
 def test_refresh_matches_policy_step_and_gather(E, S, chunks, id64, monkeypatch):
-    """One-launch refreshes (one workgroup, fewer than the tiles, more than the CUs) beside the
-    separate calls on a twin, over steps with no, some and all slots replaced, read-through
-    steps and pending prefetches to settle; state, slot ids and slot bytes after every step."""
+    """One-launch refreshes (one workgroup, fewer than the tiles, the most) and two-launch ones
+    beside the separate calls on a twin, over steps with no, some and all slots replaced and
+    pending prefetches to settle; state, slot ids and slot bytes after every step."""
     from types import SimpleNamespace
 
     from vllm_expert_cache.cache import ExpertSlotCache

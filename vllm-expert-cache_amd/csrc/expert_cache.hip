@@ -267,6 +267,7 @@ int expert_cache_refresh(const expert_cache_layer* c, const void* ids, int id_by
   // ids that are rewritten in place take two launches.
   const long long id_range = (long long)mk * id_bytes;
   if (c->E <= kGatherThreads && c->S <= kGatherThreads &&
+      (long long)c->chunks * c->lanes <= kRefreshGroups &&
       !ranges_meet(ids, id_range, out, id_range)) {
     if (id_bytes == 8)
       hipLaunchKernelGGL((refresh_k<8>), grid, block, 0, stream, EC_STEP_ARGS(a), a, g,

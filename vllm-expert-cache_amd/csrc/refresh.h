@@ -28,6 +28,13 @@ namespace ec {
 // The gather's tiles take 256 threads, so the step has four waves: E and S up to 256.
 constexpr int kRefreshWaves = kGatherThreads / kWave;
 
+// Largest grid that refreshes in one launch. The arrivals are atomics on one word, about
+// 10 ns each, which the copy of a small expert does not hide. Measured on MI355X, us a launch
+// with one 4 KB insert at 128 experts and 64 slots, one launch / two: 32 workgroups 5.0 / 5.8,
+// 128 5.6 / 5.8, 160 5.9 / 5.9, 192 6.3 / 5.9, 256 7.0 / 5.8, 1024 15.5 / 5.9; a 1 MB insert,
+// whose copy hides them, 23.8 / 26.1 at 128.
+constexpr long long kRefreshGroups = 128;
+
 template <int IDB>
 __global__ __launch_bounds__(kGatherThreads) void refresh_k(EC_STEP_PARAMS, ManageArgs rest,
                                                             GatherArgs g, unsigned* arrived) {
