@@ -213,3 +213,57 @@ def test_refresh_in_place(id64):
         for f in ("table", "slot_expert", "slot_stamp", "routed", "step", "miss", "n_miss"):
             assert torch.equal(getattr(one, f), getattr(two, f)), (t, f)
         assert torch.equal(one.slots["w"], two.slots["w"]), t
+
+
+def _prefetch_step(st, ref, pred, budget, tag):
+    """expert_cache_prefetch into the layer's own miss list, against the oracle's."""
+    d = torch.as_tensor(pred, device=gu.DEV)
+    assert gu.lib().expert_cache_prefetch(
+        gu.ptr(d), len(pred), st.E, st.S, budget, st.row("table", 0), st.row("map_cold", 0),
+        st.row("slot_expert", 0), st.row("slot_stamp", 0), st.row("routed", 0),
+        st.row("miss", 0), st.row("n_miss", 0), gu.stream()) == 0
+    assert ref.prefetch(pred, budget) == 0
+    torch.cuda.synchronize()
+    _check_state(st, ref, tag + " (prefetch)")
+
+
+@pytest.mark.parametrize("E,S", [(64, 40), (128, 100), (256, 200), (512, 300), (1024, 900),
+                                 (1300, 1000)])
+@pytest.mark.parametrize("kind", ["one high", "half high", "all high", "spread", "one old",
+                                  "half old", "past 43 bits"])
+@pytest.mark.parametrize("policy", [0, 1])
+def test_stamps_far_apart(E, S, kind, policy):
+    """Evictable slots without a 32-bit key: above all keys (they are victims only where too
+    few others are), below them (the keys start again from the smallest stamp), too few keys
+    within reach of the smallest, and stamps that have none at all. Few and many victims, in
+    the policy step and the prefetch step."""
+    rng = np.random.default_rng(E + S + len(kind))
+    for t, misses in enumerate([1, 3, 30, min(100, E - S)]):
+        near, step = rng.integers(1, 50, size=S), 1 << 20
+        stamps, pick = near.copy(), rng.permutation(S)
+        if kind == "one high":
+            stamps[pick[0]] += 1 << 40
+        elif kind == "half high":
+            stamps[pick[::2]] += 1 << 40
+        elif kind == "all high":
+            stamps += 1 << 40
+        elif kind == "spread":
+            stamps = (1 + pick) << 27
+        elif kind == "past 43 bits":
+            stamps[pick[:3]] = [1 << 43, 1 << 62, -5]
+        else:  # stamps a long way back from the step
+            step = (1 << 40) + 100
+            stamps = near + (1 << 40)
+            old = pick[:1] if kind == "one old" else pick[::2]
+            stamps[old] = near[old]
+        experts = rng.choice(E, S, replace=False)
+        st, ref = _device_state(E, S, S, experts, rng.permutation(S), stamps)
+        st.step[0] = step
+        ref.step[:] = step
+        for n in range(3):
+            cold = np.nonzero(ref.table < 0)[0]
+            ids = rng.permutation(cold)[:misses].astype(np.int32)
+            tag = f"E={E} S={S} {kind} policy={policy} misses={misses} step {n}"
+            if t % 2 == n % 2:
+                _prefetch_step(st, ref, rng.permutation(cold)[:misses].astype(np.int32), S, tag)
+            _step(st, ref, ids, S, policy, 0, False, tag)

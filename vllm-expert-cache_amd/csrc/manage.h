@@ -20,8 +20,9 @@
 //    wave takes the minimum of all keys once per insert where inserts are few; otherwise
 //    every wave sorts its 64 keys in registers and the first wave merges the sorted lists
 //    down to the 64 smallest, or, for more victims than that, a key's rank is found by a
-//    binary search in each list. Stamps too far apart for 32 bits are ranked on the 64-bit
-//    keys by counting.
+//    binary search in each list. A stamp too far above the others for a 32-bit key needs
+//    none while enough slots have one; where one lies below the keys they are counted again
+//    from the smallest, and only where that leaves too few are 64-bit keys ranked by counting.
 //
 // Measured on MI355X, us for a graph of 48 launches, against a one-wave kernel that held up to
 // 16 slots and 8 experts a lane: 128 experts, 64 slots, 8 ids 111 -> 99; 256, 192, 128 ids,
@@ -69,7 +70,7 @@ struct ManageLds {
   int ins[T];           // slot -> insert it takes, or -1
   int mis[T];           // insert r -> missing expert
   int vic[T];           // insert r -> slot, where the caller asks for it
-  long long key64[T];   // 64-bit victim keys, where the stamps need them
+  alignas(16) long long key64[T];  // 64-bit victim keys, where the stamps need them
   long long wmin[W];
   int wsum[2][W], wev[W];
 };
@@ -132,6 +133,23 @@ __device__ __forceinline__ unsigned victim_key32(long long stamp, long long base
 template <int W>
 __device__ __forceinline__ int few_inserts(int S) {
   return W == 1 ? 3 : 2 + S / 128;
+}
+
+// The smallest stamp above zero among the slots `ev` of the workgroup; negative where one of
+// those slots has a stamp without a 32-bit key whatever the base. All threads call it.
+template <int W, bool GLOBAL_E>
+__device__ __forceinline__ long long smallest_stamp(ManageLds<W, GLOBAL_E>& L, bool ev,
+                                                    long long stamp) {
+  long long low = kKeyMax;
+  if (ev) low = stamp < -1 || stamp >= 1ll << 43 ? -1 : stamp > 0 ? stamp : kKeyMax;
+  low = wave_min_i64(low);
+  if constexpr (W > 1) {
+    if (__lane_id() == 0) L.wmin[wave_index()] = low;
+    lds_sync();
+#pragma unroll 1
+    for (int w = 0; w < W; ++w) low = min(low, L.wmin[w]);
+  }
+  return low;
 }
 
 __device__ __forceinline__ long long uniform_i64(long long v) {
@@ -317,9 +335,9 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const int mine = (int)(__popcll(ballot(fb != 0)) << 16 | __popcll(mask));
     int before = 0, all = mine;
     if constexpr (PF) {
-      // the prefetch step has no step counter to measure stamps from: their maximum serves
-      const long long top = wave_min_i64(~(slot ? sp : 0));
-      if (lane == 0) L.wmin[wave] = top;
+      // the prefetch step has no step counter to measure stamps from
+      const long long low = wave_min_i64(slot && sp > 0 ? sp : kKeyMax);
+      if (lane == 0) L.wmin[wave] = low;
     }
     if constexpr (W > 1) {
       if (lane == 0) L.wsum[0][wave] = mine;
@@ -349,8 +367,8 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     n = wave_incl_scan(n);
     if (lane == kWave - 1) L.wsum[1][wave] = n;
     if constexpr (PF) {
-      const long long top = wave_min_i64(~(slot ? sp : 0));
-      if (lane == 0) L.wmin[wave] = top;
+      const long long low = wave_min_i64(slot && sp > 0 ? sp : kKeyMax);
+      if (lane == 0) L.wmin[wave] = low;
     }
     lds_sync();
     int before;
@@ -433,17 +451,37 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     const bool ev = slot & !fx;
     long long base = 1;
     if constexpr (PF) {
-      long long top = kKeyMax;
-      for (int w = 0; w < W; ++w) top = min(top, L.wmin[w]);
-      base = max(1ll, ~top - ((1ll << (32 - SB)) - 8));
+      base = kKeyMax;
+      for (int w = 0; w < W; ++w) base = min(base, L.wmin[w]);
     } else {
       if (lru) base = max(1ll, st - ((1ll << (32 - SB)) - 8));
     }
     bool fits;
     unsigned key = victim_key32<SB>(sp, base, tid, fits);
-    if (!ev) key = kKeyNone;
-    const int nev_wave = (int)__popcll(ballot(ev)) | (ballot(ev & !fits) ? 1 << 16 : 0);
+    if (!(ev & fits)) key = kKeyNone;
+    // Evictable slots, and from bit 16 those among them whose stamp is too far above `base`
+    // for a key: it is above all stamps that have one, so such a slot is no victim where
+    // `nact` others have keys. (Without ageing a popular expert's count passes 2^22 in a
+    // layer of more than 512 slots; with every such step ranked by counting, one insert at
+    // 900 slots took 22 us on MI355X, and takes 4.) From bit 27 waves with a stamp below
+    // `base`, or without a key at any base: then the upper half alone exceeds the slots.
+    int nev_wave = (int)__popcll(ballot(ev));
+    const unsigned long long far = ballot(ev & !fits);
+    if (__builtin_expect(far != 0, 0)) {
+      const unsigned long long above = ballot(ev & !fits & (sp > base) & (sp < 1ll << 43));
+      nev_wave |= (int)((unsigned)__popcll(above) << 16 | (above != far ? 1u << 27 : 0u));
+    }
     int nev = nev_wave;
+    const auto keyed = [&] { return nact <= (nev & 0xFFFF) - (int)((unsigned)nev >> 16); };
+    // Keys again, counted from the smallest evictable stamp: under LRU, for a slot that was
+    // last used millions of steps ago (one insert at 900 slots 9.5 us, by counting 22).
+    const auto rebase = [&]() -> bool {
+      base = smallest_stamp(L, ev, sp);
+      key = victim_key32<SB>(sp, base, tid, fits);
+      if (!ev || !fits) key = kKeyNone;
+      return base > 0;
+    };
+    bool by_count = false;
     const bool few = nins <= few_inserts<W>(S);
     int r = -1;  // insert this thread's slot takes
     if constexpr (W > 1) {
@@ -456,7 +494,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
       int before;
       wave_sums<W>(L.wev, wave, before, nev);
       nact = min(nins, nev & 0xFFFF);
-      if (__builtin_expect(nev <= 0xFFFF && nact <= kWave, 1)) {
+      if (__builtin_expect(keyed() && nact <= kWave, 1)) {
         if (wave == 0) {
           unsigned v = sorted;  // to become, in lane i, the i-th smallest key
           if (few) {
@@ -484,10 +522,22 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
         }
         lds_sync();
         r = L.ins[tid];
-      } else if (nev <= 0xFFFF) {
+      } else {
+        unsigned mine = sorted;
+        if (!keyed()) {
+          by_count = !rebase();
+          mine = wave_sort(key);
+          L.key[tid] = mine;
+          const int n = (int)__popcll(ballot(key != kKeyNone));
+          if (lane == 0) L.wev[wave] = n;
+          lds_sync();
+          int keys;
+          wave_sums<W>(L.wev, wave, before, keys);
+          by_count |= keys < nact;
+        }
         // more victims than lanes: rank of this thread's sorted key, the keys below it in
         // every wave's sorted list (in its own, its lane), four lists searched at a time
-        if (sorted != kKeyNone) {
+        if (!by_count && mine != kKeyNone) {
           int rank = 0;
           const int lists = (S + kWave - 1) / kWave;
 #pragma unroll 1
@@ -497,16 +547,16 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
             for (int step = 32; step > 0; step >>= 1) {
 #pragma unroll
               for (int q = 0; q < 4; ++q)
-                if (q < W && L.key[min(w0 + q, W - 1) * kWave + p[q] + step - 1] < sorted)
+                if (q < W && L.key[min(w0 + q, W - 1) * kWave + p[q] + step - 1] < mine)
                   p[q] += step;
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               if (q < W && w0 + q < lists)
-                rank += p[q] + (L.key[(w0 + q) * kWave + p[q]] < sorted ? 1 : 0);
+                rank += p[q] + (L.key[(w0 + q) * kWave + p[q]] < mine ? 1 : 0);
             }
           }
-          if (rank < nact) L.ins[sorted & (T - 1)] = rank;
+          if (rank < nact) L.ins[mine & (T - 1)] = rank;
         }
         // the slots of a wave's keys are its own threads': ordered within the wave
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
@@ -514,7 +564,9 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
       }
     } else {
       nact = min(nins, nev & 0xFFFF);
-      if (nev <= 0xFFFF) {
+      if (__builtin_expect(!keyed(), 0))
+        by_count = !rebase() || (int)__popcll(ballot(key != kKeyNone)) < nact;
+      if (!by_count) {
         if (few) {
 #pragma unroll 1
           for (int i = 0; i < nact; ++i) {
@@ -533,15 +585,21 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
         }
       }
     }
-    if (__builtin_expect(nev > 0xFFFF, 0)) {
-      // stamps too far apart for 32-bit keys: rank by counting on the 64-bit ones
+    if (__builtin_expect(by_count, 0)) {
+      // stamps too far apart for 32-bit keys: rank by counting on the 64-bit ones, two a read
+      // (entries past S hold the largest)
+      typedef long long i64x2 __attribute__((ext_vector_type(2)));
       const long long k64 = ev ? victim_key(sp, tid) : kKeyMax;
       L.key64[tid] = k64;
       lds_sync();
       if (ev) {
+        const i64x2* pair = reinterpret_cast<const i64x2*>(L.key64);
         int rank = 0;
 #pragma unroll 4
-        for (int i = 0; i < S; ++i) rank += L.key64[i] < k64 ? 1 : 0;
+        for (int i = 0; i < (S + 1) / 2; ++i) {
+          const i64x2 k = pair[i];
+          rank += (k.x < k64) + (k.y < k64);
+        }
         if (rank < nact) r = rank;
       }
     }
