@@ -9,9 +9,9 @@ the LDS table), both victim searches (few inserts: wave-min; many: threshold sel
 32- and 64-bit stamp spreads), insert budgets of 0, 1 and S, and predictions that are right,
 partly wrong or all wrong (ids outside [0, E) included).
 
-End to end: the prefetched copy runs on a side stream while the current stream proceeds;
-after the next refresh every resident slot must hold its expert's bytes, eagerly and in
-HIP-graph replays checked against an eager twin.
+End to end: the prefetched copy runs on a side stream while the current stream proceeds (in a
+graph capture, on the current stream); after the next refresh every resident slot must hold
+its expert's bytes, eagerly and in HIP-graph replays checked against an eager twin.
 """
 from __future__ import annotations
 

@@ -21,7 +21,8 @@ without talking to each other.
 A caller that can predict a layer's next routing (for instance from the previous layer's
 hidden state) calls `prefetch` early: the install-only policy step runs on the current
 stream and the copy of the predicted experts on a side stream, overlapping what follows;
-the layer's next `refresh` waits for that copy before its own gather. With `along=` another
+the layer's next `refresh` waits for that copy before its own gather. In a graph capture the
+copy stays on the current stream (`_copy_prefetched` says why). With `along=` another
 layer's cache, the prefetch step waits for that layer's next `refresh` and runs inside the
 same launch as its policy step (expert_cache_manage_remap_prefetch), one stream node instead
 of two. README.md:392-394 of the reference names prefetch as the path's next step.
@@ -256,7 +257,8 @@ class ExpertSlotCache:
         advance, resident predictions untouched, at most `max_inserts` installs, which
         defaults to S and is capped there) runs on the current stream. The copy of what it
         installed runs on the device's side stream (expert_cache_gather_live), so it
-        overlaps whatever the current stream does next. This layer's next `refresh` settles
+        overlaps whatever the current stream does next, except in a graph capture, where it
+        stays on the current stream. This layer's next `refresh` settles
         the prediction: routed experts stay, the others are dropped and their copy stops;
         that `refresh`, or `join`, makes the current stream wait for the copy. Returns
         False, and does nothing, when the prediction has more ids than there are slots.
@@ -316,8 +318,19 @@ class ExpertSlotCache:
         other.prefetch(pred, budget)
 
     def _copy_prefetched(self) -> None:
-        """Fork the copy of what the prefetch step just installed onto the side stream."""
+        """Fork the copy of what the prefetch step just installed onto the side stream.
+
+        Not in a graph capture: there the copy follows on the current stream. A process that
+        captured windows of eight steps of four layers, each layer's prefetch forked, beside a
+        matrix product a layer, ended with glibc's "corrupted double-linked list" (host heap)
+        in the third of such graphs, and no mistake that would explain it has been found in
+        this library. Until one is, captured graphs hold no fork of its making."""
         cur = torch.cuda.current_stream(self.table.device)
+        with torch.cuda.device(self.table.device):
+            capturing = torch.cuda.is_current_stream_capturing()
+        if capturing:
+            self._gather(self._gather_calls, self.pf_miss, self.pf_n_miss, cur.cuda_stream)
+            return
         side = _side_stream(self.table.device)
         if self._pf_done is None:  # two events per cache, re-recorded every prefetch
             self._pf_fork, self._pf_done = torch.cuda.Event(), torch.cuda.Event()
