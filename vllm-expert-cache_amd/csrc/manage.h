@@ -169,7 +169,6 @@ __device__ __forceinline__ void args_in_sgprs(const ManageArgs& a) {
 // What one thread (expert `tid`, slot `tid`) has to store for a step. A kernel whose
 // workgroups all run the step has one of them store it, once all have read the state.
 struct StepStores {
-  bool served;      // past the read-through check
   bool inserting;   // there were misses to insert, whether or not slots for them
   int routed;       // the expert's flag
   int miss;         // the expert's index in the miss list, or -1
@@ -188,6 +187,7 @@ struct StepStores {
 //          wave, before the step's own, and before the step returns;
 //  kDefer  the step's global stores go into `stores` (and the inserts' slots to L.vic)
 //          instead of to memory, and every wave's loads have returned before the step does.
+//          Such a step is always served: max_distinct is not looked at.
 struct PlainStep {
   static constexpr bool kEarly = false, kDefer = false;
   __device__ __forceinline__ void early() const {}
@@ -319,7 +319,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
   if constexpr (!GLOBAL_E) L.tab[tid] = tv;  // entries past E are written too: nothing reads them
   if constexpr (kDefer) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   step_sync<GLOBAL_E>();
-  StepStores keep{false, false, 0, -1, -1, -1, -1, 0, false, false, 0, 0, 0, 0};
+  StepStores keep{false, 0, -1, -1, -1, -1, 0, false, false, 0, 0, 0, 0};
 
   // ---- distinct count (the caller's `routed` is left holding the flags); hits mark their
   // ---- slot; misses enumerate in ascending expert id ----------------------------------
@@ -354,7 +354,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     distinct = all >> 16;
     total = all & 0xFFFF;
     const int j = (before & 0xFFFF) + __popcll(mask & lanes_below());
-    if (m && j < a.max_inserts && distinct <= a.max_distinct) {
+    if (m && j < a.max_inserts && (kDefer || distinct <= a.max_distinct)) {
       L.mis[j] = tid;
       if constexpr (kDefer)
         keep.miss = j;
@@ -397,11 +397,9 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     }
   }
   const long long st = uniform_i64(st_v) + 1;
-  if (__builtin_expect(distinct > a.max_distinct, 0)) {  // wide step: read through, nothing else changes
-    if constexpr (kDefer) {
-      keep.step = st;
-      caller.stores = keep;
-    } else if (tid == 0) {
+  // wide step: read through, nothing else changes
+  if (!kDefer && __builtin_expect(distinct > a.max_distinct, 0)) {
+    if (tid == 0) {
       if constexpr (!PF) a.step[0] = st;
       a.n_miss[0] = 0;
     }
@@ -634,7 +632,6 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     }
   }
   if constexpr (kDefer) {
-    keep.served = true;
     keep.inserting = nins > 0;
     keep.moved = slot && moved;
     keep.aged = slot && aged;
@@ -657,24 +654,22 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
 __device__ __forceinline__ void store_step(const ManageArgs& a, const StepStores& s) {
   const int tid = threadIdx.x;
   if (tid < a.E) a.routed[tid] = (unsigned char)s.routed;
-  if (s.served) {
-    if (s.miss >= 0) a.miss[2 * s.miss] = tid;
-    if (s.dropped >= 0) {
-      a.table[s.dropped] = -1;
-      a.map_cold[s.dropped] = s.dropped;
-    }
-    if (s.insert >= 0) {
-      if (s.evicted >= 0) {
-        a.table[s.evicted] = -1;
-        a.map_cold[s.evicted] = s.evicted;
-      }
-      a.table[s.expert] = tid;
-      a.map_cold[s.expert] = -1;
-      a.miss[2 * s.insert + 1] = tid;
-    }
-    if (s.aged) a.slot_stamp[tid] = s.slot_stamp;
-    if (s.moved) a.slot_expert[tid] = s.slot_expert;
+  if (s.miss >= 0) a.miss[2 * s.miss] = tid;
+  if (s.dropped >= 0) {
+    a.table[s.dropped] = -1;
+    a.map_cold[s.dropped] = s.dropped;
   }
+  if (s.insert >= 0) {
+    if (s.evicted >= 0) {
+      a.table[s.evicted] = -1;
+      a.map_cold[s.evicted] = s.evicted;
+    }
+    a.table[s.expert] = tid;
+    a.map_cold[s.expert] = -1;
+    a.miss[2 * s.insert + 1] = tid;
+  }
+  if (s.aged) a.slot_stamp[tid] = s.slot_stamp;
+  if (s.moved) a.slot_expert[tid] = s.slot_expert;
   if (tid == 0) {
     a.step[0] = s.step;
     a.n_miss[0] = s.nact;

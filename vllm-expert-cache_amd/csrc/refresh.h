@@ -9,9 +9,14 @@
 //  * A step that inserts nothing is stored by the first workgroup at once. It changes stamps
 //    and flags, and takes unrouted experts of dropped prefetches out of the table; whether
 //    there is anything to insert depends on the ids and their table entries alone, so a
-//    workgroup that reads the state late finds the same.
+//    workgroup that reads the state late finds the same. That holds because `out` does not
+//    overlap the ids, and because nothing but the routed experts' entries decides: no step
+//    reads through (max_distinct is min(E, ids)) and the insert budget is S, so a step without
+//    inserts is one without misses.
 //  * A step that inserts is stored by the last workgroup to have read the state (they count
-//    themselves in `arrived`), after its share of the copy, when its ticket has come back.
+//    themselves in `arrived`), after its share of the copy, when its ticket has come back. A
+//    workgroup takes its ticket after the step, whose second sync waits for all of its loads
+//    of the state (DeferredStep).
 //    Counting at every step, before it is known whether it inserts, put the ticket's round
 //    trip (over a microsecond) into the steps that insert nothing and gained nothing.
 //
