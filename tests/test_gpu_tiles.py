@@ -157,6 +157,53 @@ def test_refresh_matches_policy_step_and_gather(E, S, chunks, id64, monkeypatch)
             assert torch.equal(one.slots[n], two.slots[n]), (t, n)
 
 
+@pytest.mark.parametrize("E,S", [(60, 64), (128, 100), (256, 256), (200, 90)])
+@pytest.mark.parametrize("chunks,lanes", [(32, 1), (16, 2), (3, 5)])
+@pytest.mark.parametrize("id64", [False, True])
+def test_refresh_with_more_ids_than_threads(E, S, chunks, lanes, id64, monkeypatch):
+    """The one launch's four waves over several hundred to a few thousand ids, on a 16-byte
+    boundary and one id past it, on grids of one and of several lanes, beside the separate
+    calls on a twin: a cold start, steps whose experts are all resident, new experts, and ids
+    that cover every expert."""
+    from types import SimpleNamespace
+
+    from vllm_expert_cache.cache import ExpertSlotCache
+
+    monkeypatch.setenv("EXPERT_CACHE_CHUNKS", str(chunks))
+    monkeypatch.setenv("EXPERT_CACHE_LANES", str(lanes))
+    rng = np.random.default_rng(E + S + chunks)
+    owner = SimpleNamespace(a=gu.pinned(E * 12304).view(E, 12304),
+                            b=gu.pinned(E * 80).view(E, 80))
+    for t in vars(owner).values():
+        gu.fill_random(t.view(-1), int(rng.integers(1 << 30)))
+    one, two = (ExpertSlotCache(owner, list(vars(owner)), E, S, gu.DEV) for _ in range(2))
+    for c in (one, two):
+        c.policy, c.decay = 1, 2
+        for t in c.slots.values():
+            t.zero_()
+    two._layer_plan = lambda: (None, None)  # the separate calls
+    dt = torch.int64 if id64 else torch.int32
+    for t, mk in enumerate([257, 300, 300, 1000, 1025, 2600, 3001, 4096, 700]):
+        if t in (2, 4):
+            some = np.nonzero(one.table.cpu().numpy() >= 0)[0]  # resident: nothing to insert
+        else:
+            some = rng.permutation(E)[:E if t == 6 else min(E, S // 2 + 1)]
+        ids = rng.choice(some, mk)
+        ids[:2] = -1, E + 3
+        buf = torch.zeros(mk + 4, device=gu.DEV, dtype=dt)
+        ids_dev = buf[t % 2:t % 2 + mk]
+        ids_dev.copy_(torch.as_tensor(rng.permutation(ids)))
+        outs = [c.refresh(ids_dev) for c in (one, two)]
+        torch.cuda.synchronize()
+        assert torch.equal(*outs), t
+        assert int(one.arrived) == 0
+        for f in ("table", "map_cold", "slot_expert", "slot_stamp", "routed", "step", "miss",
+                  "n_miss"):
+            assert torch.equal(getattr(one, f), getattr(two, f)), (t, f)
+        for n in one.names:
+            assert torch.equal(one.slots[n], two.slots[n]), (t, n)
+
+
 def test_refresh_in_a_graph():
     """Captured refreshes of two layers, replayed with the eager twin's steps between."""
     from types import SimpleNamespace
