@@ -4,9 +4,9 @@ prefetch -> refresh sequence through the side stream.
 Kernel parity: each step runs prefetch(prediction) then manage(routing), the plugin's
 order, on one layer's state; after every call the miss list, n_miss and the full state
 (table, map_cold, slot_expert, slot_stamp, step) must equal the oracle's, bit for bit. The
-cases reach every launch variant (slots per lane 1-16, table chunks 1-8, experts beyond
-the LDS table), both victim searches (few inserts: wave-min; many: threshold select, with
-32- and 64-bit stamp spreads), insert budgets of 0, 1 and S, and predictions that are right,
+cases reach every launch variant (workgroups of 1 to 16 waves, experts beyond the 1024 of the
+LDS table), both victim searches (few inserts: repeated minimum; many: sorted keys; stamps
+that fit 32-bit keys and stamps that do not), insert budgets of 0, 1 and S, and predictions that are right,
 partly wrong or all wrong (ids outside [0, E) included).
 
 End to end: the prefetched copy runs on a side stream while the current stream proceeds (in a
@@ -38,6 +38,8 @@ CASES = [
     ("e256-s128", 256, 128, 128, 128, LFU, 64, 0.7, None),
     ("e512-s257", 512, 257, 50, 64, LRU, 0, 0.6, None),
     ("e1000-s1024", 1000, 1024, 200, 1024, LFU, 3, 0.5, None),
+    ("e1024-s300", 1024, 300, 64, 300, LFU, 3, 0.6, None),  # the most experts in LDS
+    ("e1025-s1024", 1025, 1024, 64, 1024, LFU, 3, 0.6, None),
     ("e5000-s300", 5000, 300, 64, 300, LRU, 0, 0.6, None),
     ("e128-s16-budget1", 128, 16, 8, 1, LFU, 64, 0.7, None),
     ("e128-s16-budget0", 128, 16, 8, 0, LRU, 64, 0.7, None),

@@ -6,8 +6,8 @@ overlap check must accept arrays that touch without overlapping). Step t runs la
 t % 2's policy step and remap and the other layer's prefetch of its next routing in one
 launch, so each layer alternates prefetch -> manage, the plugin's order. After every launch
 both layers' miss lists, prefetch miss lists, slot ids and full state must equal the
-oracle's, bit for bit. The cases reach every launch variant (slots per lane 1-16, table
-chunks 1-8, experts beyond the LDS table), int32 and int64 routing ids, insert budgets of
+oracle's, bit for bit. The cases reach every launch variant (workgroups of 1 to 16 waves,
+experts beyond the 1024 of the LDS table), int32 and int64 routing ids, insert budgets of
 0, 1 and S, and predictions that are right, partly wrong or all wrong.
 
 Cache level: a two-layer decode with the prefetch staged along the other layer's refresh
@@ -41,6 +41,8 @@ CASES = [
     ("e256-s128-i64", 256, 128, 128, 128, LFU, 64, 0.7, None, 8),
     ("e512-s257", 512, 257, 50, 64, LRU, 0, 0.6, None, 4),
     ("e1000-s1024", 1000, 1024, 200, 1024, LFU, 3, 0.5, None, 4),
+    ("e1024-s300", 1024, 300, 64, 300, LFU, 3, 0.6, None, 4),
+    ("e1025-s1024", 1025, 1024, 64, 1024, LFU, 3, 0.6, None, 4),
     ("e5000-s300", 5000, 300, 64, 300, LRU, 0, 0.6, None, 8),
     ("e128-s16-budget1", 128, 16, 8, 1, LFU, 64, 0.7, None, 4),
     ("e128-s16-budget0", 128, 16, 8, 0, LRU, 64, 0.7, None, 4),

@@ -8,8 +8,7 @@ expert_cache_prefetch call, then runs a fixed sequence through one entry point: 
 that reads through (pending installs must survive it), a served step on an LFU ageing step
 with other misses (a confirmed install must end at stamp 1), and a few more steps. Every
 field of the state, the miss list and the slot ids must equal the oracle's after each call.
-Shapes cover one slot per lane, eight slots per lane with the table beyond the registers,
-and experts beyond the LDS table.
+Shapes cover workgroups of one wave and of sixteen, and experts beyond the LDS table.
 """
 from __future__ import annotations
 

@@ -2,8 +2,9 @@
 //
 // Argument checks run on the host before any HIP call and return -1, exactly where the
 // reference's C-ABI does (kernels/expert_cache.hip:596-598, :616-618, :631-634); otherwise
-// each entry point launches one kernel (the fused one, for prefill chunks, two) on the
-// caller's stream and returns hipGetLastError().
+// each entry point launches one kernel on the caller's stream (two: the fused one for prefill
+// chunks, and the refresh above 256 experts or slots, on large grids, or where the slot ids
+// overwrite the routing ids) and returns hipGetLastError().
 // The library keeps no state and allocates nothing.
 #include <hip/hip_runtime.h>
 
