@@ -61,6 +61,21 @@ def test_policy_step_at_every_width(E, S, policy):
         _step(st, ref, ids, S, policy, 3, t % 2 == 1, f"E={E} S={S} policy={policy} step {t}")
 
 
+@pytest.mark.parametrize("E,S", [(8, 4), (64, 40), (128, 64), (500, 200), (1100, 300)])
+@pytest.mark.parametrize("policy", [0, 1])
+def test_more_experts_routed_than_slots(E, S, policy):
+    """Misses with few or no slots to evict: the slots' experts are all routed, or all but one
+    or two, while several or most of the others miss."""
+    rng = np.random.default_rng(E)
+    st, ref = _device_state(E, S, S, rng.choice(E, S, replace=False), rng.permutation(S),
+                            rng.integers(0, 5, size=S))
+    for t, (kept, missing) in enumerate([(S, 1), (S, 4), (S, E), (S - 1, 2), (S - 2, E), (S, E)]):
+        cold, warm = np.nonzero(ref.table < 0)[0], np.nonzero(ref.table >= 0)[0]
+        ids = np.concatenate([rng.permutation(warm)[:kept], rng.permutation(cold)[:missing]])
+        _step(st, ref, rng.permutation(ids).astype(np.int32), S, policy, 2, t % 2 == 1,
+              f"E={E} S={S} policy={policy} step {t}")
+
+
 @pytest.mark.parametrize("S,bits", [(40, 26), (100, 25), (200, 24), (500, 23), (1000, 22)])
 @pytest.mark.parametrize("policy", [0, 1])
 @pytest.mark.parametrize("misses", [3, 30])

@@ -565,7 +565,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
       if (__builtin_expect(!keyed(), 0))
         by_count = !rebase() || (int)__popcll(ballot(key != kKeyNone)) < nact;
       if (!by_count) {
-        if (few) {
+        if (nact <= few_inserts<W>(S)) {
 #pragma unroll 1
           for (int i = 0; i < nact; ++i) {
             const unsigned m = wave_min_u32(key);
