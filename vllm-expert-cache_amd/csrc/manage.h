@@ -187,7 +187,6 @@ struct StepStores {
 //          wave, before the step's own, and before the step returns;
 //  kDefer  the step's global stores go into `stores` (and the inserts' slots to L.vic)
 //          instead of to memory, and every wave's loads have returned before the step does.
-//          Such a step is always served: max_distinct is not looked at.
 struct PlainStep {
   static constexpr bool kEarly = false, kDefer = false;
   __device__ __forceinline__ void early() const {}
@@ -354,7 +353,7 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     distinct = all >> 16;
     total = all & 0xFFFF;
     const int j = (before & 0xFFFF) + __popcll(mask & lanes_below());
-    if (m && j < a.max_inserts && (kDefer || distinct <= a.max_distinct)) {
+    if (m && j < a.max_inserts && distinct <= a.max_distinct) {
       L.mis[j] = tid;
       if constexpr (kDefer)
         keep.miss = j;
@@ -397,9 +396,15 @@ __device__ __forceinline__ void manage_step(const ManageArgs& a, ManageLds<W, GL
     }
   }
   const long long st = uniform_i64(st_v) + 1;
-  // wide step: read through, nothing else changes
-  if (!kDefer && __builtin_expect(distinct > a.max_distinct, 0)) {
-    if (tid == 0) {
+  // Wide step: read through, nothing else changes. The deferring caller's max_distinct admits
+  // every step, so its arm is not reached; but without this branch the compiler holds more of
+  // that kernel's arguments across the step than fit the SGPRs (42 of their words spilled for
+  // 26, and 32 layer-steps of 96 of 128 slots took 374 us for 367).
+  if (__builtin_expect(distinct > a.max_distinct, 0)) {
+    if constexpr (kDefer) {
+      keep.step = st;
+      caller.stores = keep;
+    } else if (tid == 0) {
       if constexpr (!PF) a.step[0] = st;
       a.n_miss[0] = 0;
     }
