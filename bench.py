@@ -5,9 +5,12 @@ Workload: 48 MoE layers x 128 W8A8 experts (4,732,928 B each: int8 w13 [1536, 20
 w2 [2048, 768], fp32 scales [1536, 1] and [2048, 1]), ~29 GB of pinned host memory, top-8
 routing at decode batch 1 (Zipf 1.1 with 0.6 per-expert repeat, one seed per layer), 64 HBM
 slots per layer, LFU with decay 64, 4096-step trace. One "step" is one decode step across
-all 48 layers: per layer, the fused policy step + remap kernel and the gather kernel, as the
-plugin launches them, captured once into a HIP graph and replayed per step (the way vLLM
-runs decode). Routing ids for the step are copied into the graph's input buffer first.
+all 48 layers: per layer expert_cache_refresh (policy step, remap and gather), as the plugin
+calls it, captured once into a HIP graph and replayed per step (the way vLLM runs decode).
+Routing ids for the step are copied into the graph's input buffer first. The figures of the
+single kernels (roofline, manage_remap_*, decode_chain, stamps) are of the same step as two
+launches, expert_cache_manage_remap and expert_cache_gather, which is what the plugin issues
+beside a prefetch and in layers too large for the one launch.
 
 Windows of the trace (4096 steps for this workload):
   timed        steps W..W+K (--warmup W, --steps K): `value`, `ms_per_step` and `roofline`
@@ -22,7 +25,7 @@ Printed (one JSON line on stdout; the run exits 1 if any verification fails):
   value        gathered bytes / wall time of the timed steps (GB/s), sources in host memory
   verified     the checks above, with what each covered
   trace_pass   whole-job GB/s, ms/step and hit rate over steps W..4096
-  roofline     the gather kernel against the measured host->device link peak: achieved
+  roofline     the gather kernel of the two-launch step against the measured host->device link peak: achieved
                host->HBM GB/s over the timed steps = algorithmic bytes / what the gather
                launches add to the decode graph's time (HIP events on the launch stream,
                node substitution: decode_chain.timed); achieved_events brackets every launch
@@ -38,7 +41,9 @@ Printed (one JSON line on stdout; the run exits 1 if any verification fails):
                stamps), manage_remap_us_per_layer_policy_graph a graph of the policy
                launches alone, and manage_remap_us_per_layer_events the event-bracketed
                upper bound
-  decode_chain the decode graph's per-node costs by substitution and by clock stamps
+  decode_chain the per-node costs of the decode graph of two launches a layer by substitution
+               and by clock stamps, and beside them the graph of refreshes
+               (refresh_us_per_layer)
   hit_rate     1 - inserts / distinct routed experts over the timed steps
   hit_rate_sweep  every slot budget x LFU/LRU over the whole trace from a cold start, with
                the per-layer range
@@ -46,6 +51,7 @@ Printed (one JSON line on stdout; the run exits 1 if any verification fails):
                core over the trace pass, and a CPU-driven cache (that policy deciding the
                misses, one hipMemcpyAsync per (miss, buffer)) on a sample of the timed steps
   prefetch     1,024 steps of the steady-state window with and without next-layer prefetch
+               (the baseline: one expert_cache_refresh a layer)
                (each layer's predicted experts installed as pending by the prefetch step
                and copied on a side stream by the live gather during an earlier layer; the
                layer's real step keeps the routed ones and drops the rest), with no model
@@ -282,6 +288,16 @@ class Layers:
             getattr(self, f).copy_(snap[f])
 
 
+def _layer(_lib, st, l, E, S, policy, decay, chunks, lanes, nm_p, arrived_p, g):
+    """Layer l as expert_cache_refresh takes it; g holds its six (dst, src, bytes)."""
+    six = ctypes.c_void_p * 6
+    return _lib.Layer(E, S, policy, decay, chunks, lanes,
+                      *(st.row(f, l) for f in ("table", "map_cold", "slot_expert",
+                                               "slot_stamp", "routed", "step", "miss")),
+                      nm_p, arrived_p, six(*g[0:18:3]), six(*g[1:18:3]),
+                      (ctypes.c_long * 6)(*g[2:18:3]))
+
+
 def main():
     args = parse()
     if args.traffic_probe:
@@ -405,11 +421,16 @@ def main():
     G_ARGS = [tuple(gather_args(l)) + (st.row("miss", l), row(nm_static, l), chunks, lanes)
               for l in range(L)]
 
+    arrived = torch.zeros((L,), dtype=torch.int32, device=dev)
+    layers = [_layer(_lib, st, l, E, S, policy, decay, chunks, lanes, row(nm_static, l),
+                     row(arrived, l), gather_args(l)) for l in range(L)]
+    R_ARGS = [(ctypes.addressof(layers[l]), row(ids_static, l), 4, mk, row(out_static, l))
+              for l in range(L)]
+
     def launch_step(stream):
         s = ctypes.c_void_p(stream.cuda_stream)
         for l in range(L):
-            rc = lib.expert_cache_manage_remap(*M_ARGS[l], s)
-            rc |= lib.expert_cache_gather(*G_ARGS[l], s)
+            rc = lib.expert_cache_refresh(*R_ARGS[l], s)
             if rc:
                 raise RuntimeError(f"launch failed rc={rc}")
 
@@ -493,6 +514,7 @@ def main():
     # ---- verification of the trace pass's slot bytes (its state is checked against the ----
     # ---- oracle in the cpu_baseline leg) -------------------------------------------------
     final = st.snapshot()
+    assert not bool(arrived.any()), "a refresh left its arrival count behind"
     t1 = time.time()
     slot_ok, resident = True, 0
     for l in range(L):
@@ -586,7 +608,7 @@ def main():
 
     # ---- the decode chain's per-node costs, by substitution --------------------------------
     chain = None if args.no_chain else chain_costs(
-        torch, lib, hold, graph, M_ARGS, gather_args, st, snaps[W], final, ids_dev,
+        torch, lib, hold, graph, M_ARGS, G_ARGS, gather_args, st, snaps[W], final, ids_dev,
         ids_static, nm_hist, miss_hist, nm[:TP], W, T, TP, late0, L, S, B_exp, chunks, lanes,
         peak, dev)
     verified["chain_rerun_state"] = None if chain is None else chain.pop("rerun_state_equal")
@@ -706,6 +728,13 @@ def main():
                      "achieved": round(achieved, 3),
                      "peak": round(peak, 3), "unit": "GB/s",
                      "frac": round(achieved / peak, 4),
+                     "chain": "policy step and gather as two launches a layer; value and "
+                              "trace_pass are one refresh a layer",
+                     "refresh_us_per_layer":
+                         None if chain is None else chain["trace_pass"]["refresh_us_per_layer"],
+                     "two_launches_us_per_layer":
+                         None if chain is None
+                         else chain["trace_pass"]["two_launches_us_per_layer"],
                      "achieved_events": round(tw["achieved"], 3),
                      "frac_events": round(tw["achieved"] / peak, 4),
                      # the metric's other two parts, as scalars beside the gather's
@@ -843,15 +872,20 @@ class Hold:
 def substitution_window(times, lo, hi, nm, L, B_exp, peak):
     """The decode chain's per-node costs over trace steps [lo, hi) from the substitution
     variants' timed chunks: times[variant] = [(c0, c1, GPU seconds of chunk [c0, c1))], with
-    variants full, gathers, gathers_again, empty+gather and policy (chain_costs); only the
-    chunks that lie inside the window count. nm[t, l] is the inserts of step t, layer l."""
+    variants full, gathers, gathers_again, empty+gather, policy and refresh (chain_costs);
+    only the chunks that lie inside the window count. nm[t, l] is the inserts of step t, layer
+    l."""
     n = hi - lo
     t = {k: sum(s for c0, c1, s in v if c0 >= lo and c1 <= hi) for k, v in times.items()}
     per = 1e6 / (n * L)
     moved = float(nm[lo:hi].sum()) * B_exp
     gather_s = t["full"] - t["policy"]
+    refresh = t.get("refresh")
     return {"trace_steps": [lo, hi],
             "ms_per_step": round(1e3 * t["full"] / n, 4),
+            "refresh_ms_per_step": None if refresh is None else round(1e3 * refresh / n, 4),
+            "refresh_us_per_layer": None if refresh is None else round(refresh * per, 3),
+            "two_launches_us_per_layer": round(t["full"] * per, 3),
             "manage_remap_us_per_layer": round((t["full"] - t["gathers"]) * per, 3),
             "noise_us_per_layer": round(abs(t["gathers_again"] - t["gathers"]) * per, 3),
             "empty_node_us": round((t["empty+gather"] - t["gathers"]) * per, 3),
@@ -864,20 +898,21 @@ def substitution_window(times, lo, hi, nm, L, B_exp, peak):
             "seconds": {k: round(v, 5) for k, v in t.items()}}
 
 
-def chain_costs(torch, lib, hold, graph, m_args, gather_args, st, snap, final, ids_dev,
+def chain_costs(torch, lib, hold, graph, m_args, g_args, gather_args, st, snap, final, ids_dev,
                 ids_static, nm_hist, miss_hist, nm, W, T, TP, late0, L, S, B_exp, chunks,
                 lanes, peak, dev):
-    """What each node of the decode graph costs inside the chain, measured by substitution:
-    the graph's step time against the same step with some of its nodes taken out or
-    replaced, each replayed over the same trace steps behind stream holds. No events sit
+    """What each node of a decode graph of two launches a layer costs inside the chain, measured
+    by substitution: the graph's step time against the same step with some of its nodes taken
+    out or replaced, each replayed over the same trace steps behind stream holds. No events sit
     between the nodes and no profiler is attached, so every figure is the chain's own.
 
-      full         the decode graph: per layer the policy+remap launch, then the gather
+      full         per layer the policy+remap launch, then the gather
       gathers      per layer only the gather, of the miss list the full graph recorded at
                    that step and layer (copied in per step, so the same bytes move)
       empty+gather per layer an empty kernel node in place of the policy launch, then the
                    same gather
       policy       per layer only the policy+remap launch
+      refresh      the decode graph that the trace pass replays: one refresh a layer
     The gathers-only variant is replayed a second time; the two replays' difference per
     layer-step (noise_us_per_layer) is the scale below which a difference means nothing.
 
@@ -888,8 +923,9 @@ def chain_costs(torch, lib, hold, graph, m_args, gather_args, st, snap, final, i
       gather per launch      = (full - policy) / (steps x L), and the gather's in-chain rate
                                is the gathered bytes over (full - policy).
     Each variant is timed per window: the timed steps W..T, the trace pass W..TP and its
-    second half late0..TP. The policy and full variants restart from the snapshot at step
-    W; the full variant's final state must equal the trace pass's (rerun_state_equal)."""
+    second half late0..TP. The policy, full and refresh variants restart from the snapshot at
+    step W; the final states of the last two must equal the trace pass's
+    (rerun_state_equal)."""
     i32 = torch.int32
     # recorded miss lists as gather inputs: row l = [n_miss, e0, s0, e1, s1, ...]
     rec_dev = torch.cat([nm_hist[:TP, :, None], miss_hist[:TP]], dim=2).contiguous()
@@ -919,26 +955,36 @@ def chain_costs(torch, lib, hold, graph, m_args, gather_args, st, snap, final, i
             if lib.expert_cache_manage_remap(*m_args[l], s):
                 raise RuntimeError("policy launch failed")
 
+    def pair(s):
+        for l in range(L):
+            if lib.expert_cache_manage_remap(*m_args[l], s) or \
+                    lib.expert_cache_gather(*g_args[l], s):
+                raise RuntimeError("policy or gather launch failed")
+
     g_only = capture(gathers)
     # the gathers-only variant runs twice: the two runs' difference is the substitution's
     # noise (the host link's rate varies a little from pass to pass)
     variants = {"gathers": g_only, "empty+gather": capture(lambda s: gathers(s, empty=True)),
-                "policy": capture(policy), "full": graph, "gathers_again": g_only}
+                "policy": capture(policy), "full": capture(pair), "refresh": graph,
+                "gathers_again": g_only}
     times = {}
+    rerun_equal = True
     for name, g in variants.items():
         def enqueue(t, g=g):
             ids_static.copy_(ids_dev[t], non_blocking=True)
             rec_static.copy_(rec_dev[t], non_blocking=True)
             g.replay()
 
-        if name in ("policy", "full"):
+        if name in ("policy", "full", "refresh"):
             st.restore(snap)
         times[name] = hold.time(W, TP, enqueue, cuts=(late0, T))
         log(f"decode chain, {name}: {sum(x[2] for x in times[name]):.4f} s over steps "
             f"{W}..{TP}")
-    rerun_equal = all(torch.equal(getattr(st, f), final[f]) for f in st.fields)
+        if name in ("full", "refresh"):
+            rerun_equal = rerun_equal and all(torch.equal(getattr(st, f), final[f])
+                                              for f in st.fields)
     del g_only
-    for name in ("gathers", "empty+gather", "policy", "gathers_again"):
+    for name in ("gathers", "empty+gather", "policy", "full", "gathers_again"):
         del variants[name]
 
     def window(lo, hi=TP):
@@ -946,8 +992,8 @@ def chain_costs(torch, lib, hold, graph, m_args, gather_args, st, snap, final, i
 
     out = {"timed": window(W, T), "trace_pass": window(W), "steady_state": window(late0),
            "hold": hold.record(), "rerun_state_equal": rerun_equal,
-           "manage_remap_def": f"what the policy+remap launch adds to the decode graph per "
-                               f"layer, over trace steps {W}..{TP}: the graph's time minus "
+           "manage_remap_def": f"what the policy+remap launch adds to the decode graph of two "
+                               f"launches a layer per layer, over trace steps {W}..{TP}: the graph's time minus "
                                f"that of the same graph with only its gathers (fed the "
                                f"recorded miss lists), per layer-step; no events or "
                                f"profiler in the chain (decode_chain)",
@@ -955,14 +1001,18 @@ def chain_costs(torch, lib, hold, graph, m_args, gather_args, st, snap, final, i
     tp, ss, tm = out["trace_pass"], out["steady_state"], out["timed"]
     log(f"decode chain over the timed steps {W}..{T}: gather {tm['gather_GBps']} GB/s "
         f"({tm['gather_frac']}), {tm['gather_us_per_launch']} us per launch, policy+remap "
-        f"{tm['manage_remap_us_per_layer']} us/layer")
+        f"{tm['manage_remap_us_per_layer']} us/layer; two launches a layer "
+        f"{tm['two_launches_us_per_layer']} us, one refresh {tm['refresh_us_per_layer']}")
     log(f"decode chain over steps {W}..{TP}: policy+remap {tp['manage_remap_us_per_layer']} "
         f"us/layer (noise {tp['noise_us_per_layer']}, empty node {tp['empty_node_us']}, "
         f"policy-only graph "
         f"{tp['policy_graph_us_per_layer']}), gather {tp['gather_GBps']} GB/s "
         f"({tp['gather_frac']}); steady state from {late0}: policy+remap "
         f"{ss['manage_remap_us_per_layer']} us/layer, gather {ss['gather_GBps']} GB/s "
-        f"({ss['gather_frac']}); re-run state {'equal' if rerun_equal else 'MISMATCH'}")
+        f"({ss['gather_frac']}); a layer of two launches {tp['two_launches_us_per_layer']} us, "
+        f"one refresh {tp['refresh_us_per_layer']} (steady state "
+        f"{ss['two_launches_us_per_layer']}, {ss['refresh_us_per_layer']}); re-run state "
+        f"{'equal' if rerun_equal else 'MISMATCH'}")
     return out
 
 
@@ -989,8 +1039,8 @@ def _stamps_lib():
 
 def chain_stamps(torch, np, hold, m_args, g_args, st, snap, final, ids_dev, ids_static, nm,
                  W, TP, late0, L, B_exp, grid, peak, dev):
-    """The decode chain's kernel times from inside the kernels: the decode graph rebuilt
-    with bench_stamps.so's stamped copies of the policy+remap and gather kernels (the
+    """The decode chain's kernel times from inside the kernels: the decode graph of two launches
+    a layer rebuilt with bench_stamps.so's stamped copies of the policy+remap and gather kernels (the
     product's device code between two reads of the GPU's constant-rate clock) and replayed
     over trace steps W..TP from the snapshot at W, the stamps of every launch kept. Then the
     same with the policy launches alone (back to back). Per window (the trace pass, and the
@@ -1467,7 +1517,8 @@ def _prefetch_matches(np, want, nm, miss, pn, pf_miss, final):
 
 
 PREFETCH_RUNS = (
-    {},                                                     # no prefetch
+    {},                                                     # no prefetch: the baseline
+    {"split": True},                                        # ... as two launches a layer
     {"accuracy": 1.0, "lookahead": 1, "one_launch": False},
     {"accuracy": 1.0, "lookahead": 1},
     {"accuracy": 1.0, "lookahead": 1, "late_fork": True},
@@ -1513,7 +1564,8 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
     `snap` taken at step W of the trace pass), as one captured graph per decode step.
 
     With a lookahead of d layers:
-      d = 0 (no prefetch): per layer l, manage+remap(l), gather(l), compute(l);
+      d = 0 (no prefetch): per layer l, refresh(l), compute(l), as a program without prefetch
+              has it; with "split", manage+remap(l), gather(l), compute(l);
       d >= 1: layers 0..d-1 prefetched first, then per layer l the prefetch step of layer
               l+d and manage+remap(l) -- two launches (expert_cache_prefetch, then
               expert_cache_manage_remap) or one (expert_cache_manage_remap_prefetch) --,
@@ -1531,8 +1583,8 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
     compute(l) stands in for the layer's attention and expert GEMMs: a spin of C us on one
     CU (C = 0: no compute, so prefetch has nothing to hide behind). Predictions come from
     _predictions; accuracy 1.0 is an upper bound no real predictor reaches. Each run is a
-    dict of accuracy (absent: no prefetch), lookahead, one_launch (default True), late_fork
-    (default False), pair (default False), budget (inserts per prefetch step, default S) and
+    dict of accuracy (absent: no prefetch), split (default False), lookahead, one_launch
+    (default True), late_fork (default False), pair (default False), budget (inserts per prefetch step, default S) and
     errors ("uniform", the default, or "routed").
 
     Checked: every run's per-step n_miss and miss list of each layer's real step and of its
@@ -1606,6 +1658,20 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
     gr_args = [tuple(g_args[l][:18]) + (st.row("miss", l), _row(nm_static, l), chunks, lanes)
                for l in range(L)]
 
+    from vllm_expert_cache import _lib
+    arrived = torch.zeros((L,), dtype=i32, device=dev)
+    layers = [_layer(_lib, st, l, E, S, policy, decay, chunks, lanes, _row(nm_static, l),
+                     _row(arrived, l), g_args[l]) for l in range(L)]
+
+    def refreshes(cur, spin):
+        c = ctypes.c_void_p(cur.cuda_stream)
+        for l in range(L):
+            if lib.expert_cache_refresh(ctypes.addressof(layers[l]), _row(ids_static, l), 4, mk,
+                                        _row(out_static, l), c):
+                raise RuntimeError("refresh launch failed")
+            if spin:
+                torch.cuda._sleep(spin)
+
     def launch(cur, la, one, late, budget, spin, pair=False):
         c = ctypes.c_void_p(cur.cuda_stream)
         sd = ctypes.c_void_p(side.cuda_stream)
@@ -1664,7 +1730,7 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
             q = run.get("accuracy")
             la = run.get("lookahead", 0) if q is not None else 0
             one, late = run.get("one_launch", True), run.get("late_fork", False)
-            pair = run.get("pair", False)
+            pair, split = run.get("pair", False), run.get("split", False)
             budget = run.get("budget") or S
             errors = run.get("errors", "uniform")
             pred = None if q is None else (ids_np[W:W + K].copy() if q >= 1.0 else
@@ -1683,8 +1749,11 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
             torch.cuda.synchronize()
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):
-                launch(torch.cuda.current_stream(), la, one, late, budget, int(C * cyc_per_us),
-                       pair)
+                if q is None and not split:
+                    refreshes(torch.cuda.current_stream(), int(C * cyc_per_us))
+                else:
+                    launch(torch.cuda.current_stream(), la, one, late, budget,
+                           int(C * cyc_per_us), pair)
             torch.cuda.synchronize()
             wall0 = time.perf_counter()
             a.record()
@@ -1725,12 +1794,14 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
                 used = int((routed[tt[..., None], ll[..., None], np.where(valid, fetched, 0)]
                             & valid).sum())
             ms = 1e3 * elapsed / K
-            if q is None:
+            if q is None and not split:
                 base_ms[C] = ms
             useful = (int(nm.sum()) + used) * B_exp / elapsed / 1e9
             out.append({"compute_us_per_layer": C, "predictor_accuracy": q,
                         "prediction_errors": errors if q is not None and q < 1.0 else None,
                         "lookahead_layers": la, "one_launch": one if la else None,
+                        "launches_per_layer_without_prefetch":
+                            None if q is not None else 2 if split else 1,
                         "copy_fork": (None if not la else
                                       "after the layer's gather" if late else
                                       "after every second policy launch, two layers' "
@@ -1743,7 +1814,7 @@ def prefetch_leg(torch, np, lib, ids_np, ids_dev, g_args, snap, L, E, S, mk, pol
                         "prefetch_dropped": int(pn.sum()) - used,
                         "critical_path_inserts": int(nm.sum()),
                         "real_step_hit_rate": round(1.0 - float(nm.sum()) / distinct, 5)})
-            desc = "none" if q is None else (
+            desc = ("none, two launches" if split else "none") if q is None else (
                 f"{q} ({errors} errors), lookahead {la}"
                 f"{', one launch' if one else ', two launches'}"
                 f"{', copy forked after the gather' if late else ''}"

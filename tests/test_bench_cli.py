@@ -135,7 +135,8 @@ def test_substitution_windows_count_only_their_chunks():
     nm[25:] = np.arange(4096 - 25)[:, None] % 2
     g = nm.sum(1) * B / rate + L * 1.5e-6           # gathers-only graph, per step
     per_step = {"gathers": g, "gathers_again": g, "empty+gather": g + L * 1.5e-6,
-                "full": g + L * 2.4e-6, "policy": np.full(4096, L * 2.5e-6)}
+                "full": g + L * 2.4e-6, "policy": np.full(4096, L * 2.5e-6),
+                "refresh": np.full(4096, L * 7.5e-6)}
     times = {k: [(c0, c1, float(v[c0:c1].sum())) for c0, c1 in zip(pts[:-1], pts[1:])]
              for k, v in per_step.items()}
     for lo, hi in ((5, 25), (5, 4096), (2048, 4096)):
@@ -147,6 +148,7 @@ def test_substitution_windows_count_only_their_chunks():
         assert w["manage_remap_over_empty_node_us"] == 0.9
         assert w["noise_us_per_layer"] == 0.0
         assert w["policy_graph_us_per_layer"] == 2.5
+        assert w["refresh_us_per_layer"] == 7.5
         gather_s = float((g[lo:hi] - L * 0.1e-6).sum())
         assert w["gather_GBps"] == round(float(nm[lo:hi].sum()) * B / gather_s / 1e9, 3)
         assert abs(w["gather_us_per_launch"] - gather_s * 1e6 / ((hi - lo) * L)) < 1e-3
