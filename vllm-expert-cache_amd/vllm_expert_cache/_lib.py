@@ -6,8 +6,9 @@ Same search order and same argument lists for the reference's two bound entry po
 points that replace the reference's torch remap, `expert_cache_prefetch`,
 `expert_cache_manage_remap_prefetch` (one layer's policy step with another's prefetch step
 in one launch), `expert_cache_gather_live` (the prefetch copy that stops for dropped
-predictions), and `expert_cache_refresh` (policy step, remap and gather in one call). Every call is asynchronous on the caller's stream and never reads a device
-value back, so the whole path is HIP-graph capturable.
+predictions), and `expert_cache_refresh` (policy step, remap and gather in one call). Every
+call is asynchronous on the caller's stream and never reads a device value back, so the whole
+path is HIP-graph capturable.
 
 There is no fallback: if the library or one of its symbols is missing, loading fails with
 an error that says so.

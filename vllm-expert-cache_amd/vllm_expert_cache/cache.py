@@ -10,8 +10,8 @@ expert_cache_refresh, which is in one launch
      the (expert, slot) miss list, and rewrites the routing ids into slot ids;
   2. expert_cache_gather: pulls each missing expert's slabs from host memory into its slot.
 
-Where a prefetch is staged with the step or its copy is still under way, the two are launched
-one after the other.
+Where a prefetch is staged with the step or its copy is still under way, above 256 experts or
+slots, and on gather grids above 128 workgroups, the two are launched one after the other.
 
 The fused-MoE GEMM then runs unchanged against the slot buffers with the slot ids. Nothing
 reads a device value back to the host, so the sequence is graph-capturable, and the kernels
