@@ -26,7 +26,7 @@
 //
 // Measured on MI355X, us for a graph of 48 launches, against a one-wave kernel that held up to
 // 16 slots and 8 experts a lane: 128 experts, 64 slots, 8 ids 111 -> 99; 256, 192, 128 ids,
-// 6.6 inserts a launch 246 -> 151; 512, 257, 50 ids, 2.6 inserts 274 -> 146.
+// 6.6 inserts a launch 246 -> 152; 512, 257, 50 ids, 2.6 inserts 274 -> 146.
 #pragma once
 #include <type_traits>
 
