@@ -178,8 +178,8 @@ def test_refresh_matches_policy_step_and_gather(E, S, chunks, id64, monkeypatch)
 def test_refresh_with_more_ids_than_threads(E, S, chunks, lanes, id64, monkeypatch):
     """The one launch's four waves over several hundred to a few thousand ids, on a 16-byte
     boundary and one id past it, on grids of one and of several lanes, beside the separate
-    calls on a twin: a cold start, steps whose experts are all resident, new experts, and ids
-    that cover every expert."""
+    calls on a twin: a cold start, steps whose experts are all resident, new experts, ids
+    that cover every expert, and no ids."""
     from types import SimpleNamespace
 
     from vllm_expert_cache.cache import ExpertSlotCache
@@ -198,13 +198,13 @@ def test_refresh_with_more_ids_than_threads(E, S, chunks, lanes, id64, monkeypat
             t.zero_()
     two._layer_plan = lambda: (None, None)  # the separate calls
     dt = torch.int64 if id64 else torch.int32
-    for t, mk in enumerate([257, 300, 300, 1000, 1025, 2600, 3001, 4096, 700]):
+    for t, mk in enumerate([257, 300, 300, 1000, 1025, 2600, 3001, 4096, 0, 700]):
         if t in (2, 4):
             some = np.nonzero(one.table.cpu().numpy() >= 0)[0]  # resident: nothing to insert
         else:
             some = rng.permutation(E)[:E if t == 6 else min(E, S // 2 + 1)]
         ids = rng.choice(some, mk)
-        ids[:2] = -1, E + 3
+        ids[:2] = [-1, E + 3][:mk]
         buf = torch.zeros(mk + 4, device=gu.DEV, dtype=dt)
         ids_dev = buf[t % 2:t % 2 + mk]
         ids_dev.copy_(torch.as_tensor(rng.permutation(ids)))
